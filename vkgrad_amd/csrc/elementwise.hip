@@ -293,25 +293,40 @@ struct CopyMulti {
     const uint32_t *src[MG_COPY_MAX];
     uint32_t *dst[MG_COPY_MAX];
     int64_t bytes[MG_COPY_MAX];
-    int vec[MG_COPY_MAX];
+    int vec[MG_COPY_MAX], walk[MG_COPY_MAX];
 };
-// Few workgroups that walk through the buffer together, four loads a thread: over PCIe requests in the order of their
-// addresses are worth 54 GB/s from 16 workgroups, 50 from 64 and 41 with a workgroup for every 4 KB (3 MB: 55, 60, 74 us).
+// A thread takes 16 bytes, all of a copy on their way at once.  walk: COPY_WALK workgroups go through the buffer together, four
+// loads a thread: over PCIe, requests in the order of their addresses are worth 54 GB/s from 16 workgroups, 50 from 64 and 41
+// with a workgroup for every 4 KB.  Only for aligned host memory beyond COPY_WALK_BYTES (a workgroup for every 4 KB / walking, us,
+// one copy and the wait for it: 128 KB 15.2 / 16.5, 256 KB 18.1 / 19.0, 384 KB 21.2 / 21.2, 512 KB 24.3 / 24.0, 1 MB 37.0 / 33.7, 3 MB
+// 85 / 72; between others: 3 MB of host memory that is aligned to 4 bytes 64 / 241, 6 MB in HBM 5.5 / 18.7).
+constexpr int COPY_WALK = 16;
+constexpr int64_t COPY_WALK_BYTES = 384 << 10;
 __global__ void __launch_bounds__(256) k_copy_multi(const CopyMulti a) {
     const int w = blockIdx.y;
-    const int64_t n = a.bytes[w], n16 = a.vec[w] ? n / 16 : 0, step = (int64_t)gridDim.x * 256, i0 = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    const int64_t n = a.bytes[w], i = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const uint32_t *src = a.src[w];
     uint32_t *dst = a.dst[w];
-    for (int64_t i = i0; i < n16; i += 4 * step) {
-        uint4 v[4];
+    if (a.walk[w]) {
+        if (blockIdx.x >= COPY_WALK) return;   // (the grid is that of the widest copy)
+        constexpr int STEP = COPY_WALK * 256;
+        const int64_t n16 = n / 16;
+        for (int64_t at = i; at < n16; at += 4 * STEP) {
+            uint4 v[4];
 #pragma unroll
-        for (int u = 0; u < 4; u++) v[u] = reinterpret_cast<const uint4 *>(src)[i + u * step < n16 ? i + u * step : i];
+            for (int u = 0; u < 4; u++) v[u] = reinterpret_cast<const uint4 *>(src)[at + u * STEP < n16 ? at + u * STEP : at];
 #pragma unroll
-        for (int u = 0; u < 4; u++)
-            if (i + u * step < n16) reinterpret_cast<uint4 *>(dst)[i + u * step] = v[u];
+            for (int u = 0; u < 4; u++)
+                if (at + u * STEP < n16) reinterpret_cast<uint4 *>(dst)[at + u * STEP] = v[u];
+        }
+        if (i < n % 16) reinterpret_cast<uint8_t *>(dst)[n16 * 16 + i] = reinterpret_cast<const uint8_t *>(src)[n16 * 16 + i];
+    } else if (a.vec[w] && i * 16 + 15 < n) {
+        reinterpret_cast<uint4 *>(dst)[i] = reinterpret_cast<const uint4 *>(src)[i];
+    } else {
+        for (int64_t j = i * 4; j < i * 4 + 4 && j < n / 4; j++) dst[j] = src[j];
+        if (i * 16 <= n && n < i * 16 + 16)   // the last piece: bytes behind the last whole word
+            for (int64_t j = n / 4 * 4; j < n; j++) reinterpret_cast<uint8_t *>(dst)[j] = reinterpret_cast<const uint8_t *>(src)[j];
     }
-    for (int64_t j = n16 * 4 + i0; j < n / 4; j += step) dst[j] = src[j];
-    if (i0 < n % 4) reinterpret_cast<uint8_t *>(dst)[n / 4 * 4 + i0] = reinterpret_cast<const uint8_t *>(src)[n / 4 * 4 + i0];
 }
 
 // Gradients of a list of parameters into, or back out of, a flat accumulator in one launch (an AdamW-style table: g the
@@ -437,7 +452,7 @@ int mg_ew_copy(mg_ctx *ctx, void *dst, const void *src, int64_t nbytes) {
 int mg_ew_copy_multi(mg_ctx *ctx, void *const *dst, const void *const *src, const int64_t *nbytes, int n) {
     EW_PRECHECK("mg_ew_copy_multi", dst && src && nbytes && n > 0 && n <= MG_COPY_MAX);
     CopyMulti a{};
-    int64_t widest = 1;   // workgroups of a copy: 16 where a large source is host memory, else one for every 16 KB
+    int64_t widest = 1;   // workgroups
     for (int i = 0; i < n; i++) {
         if (!dst[i] || !src[i] || !count_ok(nbytes[i]) || (((uintptr_t)dst[i] | (uintptr_t)src[i]) & 3))
             return mg::ctx_fail(MG_ERR_ARG, "mg_ew_copy_multi: bad argument");
@@ -445,16 +460,15 @@ int mg_ew_copy_multi(mg_ctx *ctx, void *const *dst, const void *const *src, cons
         a.dst[i] = (uint32_t *)dst[i];
         a.bytes[i] = nbytes[i];
         a.vec[i] = (((uintptr_t)dst[i] | (uintptr_t)src[i]) & 15) == 0;
-        int64_t blocks = (nbytes[i] + 16383) / 16384;
-        if (blocks > 16) {
+        if (a.vec[i] && nbytes[i] > COPY_WALK_BYTES) {   // (asking takes less than 0.2 us)
             hipPointerAttribute_t at{};
             const hipError_t e = hipPointerGetAttributes(&at, src[i]);
             if (e != hipSuccess) (void)hipGetLastError();
-            if (e != hipSuccess || at.type != hipMemoryTypeDevice) blocks = 16;
+            a.walk[i] = e == hipSuccess && at.type == hipMemoryTypeHost;
         }
+        const int64_t blocks = a.walk[i] ? COPY_WALK : blocks_for((nbytes[i] + 15) / 16);
         if (blocks > widest) widest = blocks;
     }
-    if (widest > 65535) widest = 65535;
     hipLaunchKernelGGL(k_copy_multi, dim3((unsigned)widest, (unsigned)n), dim3(256), 0, ctx_stream(ctx), a);
     EW_POSTCHECK("mg_ew_copy_multi");
 }
