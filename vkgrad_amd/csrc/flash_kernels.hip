@@ -28,10 +28,11 @@
 //
 // What bounds them: the exponentials and the arithmetic around them (a transcendental takes 16
 // clocks a wavefront, 256 a block of 32 x 32, as much as its MFMAs) and the latency from one to the next, not memory:
-// 96 heads x 1024 x 64 read and write 60 MB forward.  Masks are branches over whole tiles (FK_BRANCH), sums and maxima
-// trees; the sum walk takes no maximum of a tile until a sum grows large.  Measured there (bf16): forward 41.6 us (43.1 with a maximum
-// a tile, 49 with a serial one and a branch a block as well), backward 83.9 (85.5 with P narrowed twice, 99 with a mask test an element in
-// the dK / dV kernel, which the compiler made a branch an element).
+// 96 heads x 1024 x 64 read and write 60 MB forward.  Masks are branches over whole tiles (FK_BRANCH), maxima
+// trees; the sum of a row goes key by key.  Measured there (bf16, kernel by kernel): forward 41.8 us (40.5 with sums as trees and
+// no maximum of a tile until a sum reaches 2^100, which costs lse up to six bits; 48 with a serial maximum and a branch a block),
+// backward 39.5 + 49.8 (44.8 + 62 with P narrowed twice and a mask test an element in the dK / dV kernel, which the
+// compiler made a branch an element).
 // P is rebuilt twice in the backward pass, once per kernel: that costs 7 products instead of 5, but dQ needs no
 // atomics, no clear and no narrowing pass.  Three wavefronts a SIMD forward, two in the dK / dV kernel.
 #include "flash_common.h"
@@ -40,7 +41,7 @@ namespace mg {
 
 // Which head and which rows (longest first) a workgroup takes.  Consecutive workgroups fill the CUs round by round; every
 // second round is dealt out backwards, eight at a time so that a head stays on its XCD, and a CU's
-// share evens out: in order, one CU gets the longest of every round (96 heads x 1024 x 64, before the sum walk lost its maxima: 45.3 + 88.3
+// share evens out: in order, one CU gets the longest of every round (96 heads x 1024 x 64: 45.3 + 88.3
 // us in order, 43.1 + 85.5 so).
 struct FkWork {
     int bh, y;
@@ -110,28 +111,19 @@ k_flash_fwd(const FkArgs p) {
         if (j0 > i0 + 31) continue;          // every key beyond every query of this wavefront
         fk_f32x16 s[2];
         scores(kt, j0, s);
-        auto sum = [&] {
-            float v = 0.f;
-#pragma unroll
-            for (int bl = 0; bl < 2; bl++) {
-                float e[16];
-#pragma unroll
-                for (int r = 0; r < 16; r++) e[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[bl][r], c2, -m));
-                v += fk_sum16(e);
-            }
-            return v;
-        };
-        // The reference point need not be the maximum: that of the first tile that a row sees stays until a sum grows large.
-        float now = sum();
-        if (__any(!(l + now < 1.2676506e30f))) {   // 2^100; also what refers to FK_NOTHING, and NaN
-            float mt = fmaxf(fk_max16(s[0]), fk_max16(s[1]));
-            mt = fk_both(mt, [](float x, float y) { return fmaxf(x, y); }) * c2;
+        // The reference point need not be the maximum, but stays within 8 of it: further off, the exponents that matter would be
+        // held with fewer bits (a first tile 60 below the rest, a sum up to 2^100: an error of lse of 3.9e-6 for 0.8e-6).
+        float mt = fmaxf(fk_max16(s[0]), fk_max16(s[1]));
+        mt = fk_both(mt, [](float x, float y) { return fmaxf(x, y); }) * c2;
+        if (__any(mt > m + 8.f)) {
             const float mn = fmaxf(m, mt);
             l *= __builtin_amdgcn_exp2f(m - mn);
             m = mn;
-            now = sum();
         }
-        l += now;
+#pragma unroll
+        for (int bl = 0; bl < 2; bl++)
+#pragma unroll
+            for (int r = 0; r < 16; r++) l += __builtin_amdgcn_exp2f(__builtin_fmaf(s[bl][r], c2, -m));
     }
     ks.load(kb, pitch, t0 * FK_BN, T, hd, tid);
     vs.load(vb, pitch, t0 * FK_BN, T, hd, tid);
