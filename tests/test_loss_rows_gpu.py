@@ -52,3 +52,26 @@ def test_loss_with_and_without_gradients(dev, rows, stride, ncls, dtype):
                 assert np.abs(b32.download(np.float32, (rows, stride)) - dl32).max() <= 1e-6
     for b in bufs:
         b.destroy()
+
+
+@pytest.mark.parametrize("ncls,more", [(96, 700), (2000, 9000), (20000, 30000)])   # a wavefront, 256 and 1024 threads a row
+def test_impossible_classes_change_no_bit(dev, ncls, more):
+    """A thread adds its exponentials up one after the other, however many of its loads travel together: the sum, and so the loss,
+    does not depend on what follows a class."""
+    from vkgrad_amd.tkernels import make_transformer_kernels
+    TK, rows = make_transformer_kernels(dev, "bf16"), 64
+    rng = np.random.default_rng(ncls)
+    logits = np.full((rows, more), -np.inf, np.float32)
+    logits[:, :ncls] = rng.standard_normal((rows, ncls)) - np.log(ncls)
+    labels = rng.integers(0, ncls, rows).astype(np.uint32)
+    logits[np.arange(rows), labels] = 0                      # losses of about 1: their last bit is that of the sum
+    losses = []
+    for n in (ncls, more):
+        bl, by, bloss = dev.buffer(4 * rows * n, "device"), dev.buffer(4 * rows, "device"), dev.buffer(4 * rows, "device")
+        bl.upload(np.ascontiguousarray(logits[:, :n]))
+        by.upload(labels)
+        TK["softmax_ce"]([bl, by, None, None, bloss], rows, n, n)
+        losses.append(bloss.download(np.float32, (rows,)))
+        for b in (bl, by, bloss):
+            b.destroy()
+    assert np.isfinite(losses[0]).all() and np.array_equal(*losses)

@@ -807,10 +807,10 @@ __global__ void k_zero_f32(float *dst, int64_t n) {
 // a 50304-wide row in the registers of one 1024-thread workgroup, so that HBM sees it once, was slower -
 // 1.15 ms against 0.82 ms for 8192 rows: every wavefront of a CU is then in the same phase, and loads,
 // exponentials and stores no longer overlap.)  Rows whose pitch and base are 16-byte aligned move as
-// float4 / four 16-bit values, CE_ILP of them requested at once and the maximum moved once for all.
-// 32-bit sums of exponentials as before.  Measured (us, one load at a time and 256 threads for every row below a
-// vocabulary / now): 8192 x 50257 bf16 570 / 551 (4.5 TB/s), loss alone of 4096 x 50257 298 / 136 (6.0 TB/s), 2048 x 4096
-// 17.6 / 14.5, 16384 x 96 38 / 13.4.
+// float4 / four 16-bit values, CE_ILP of them requested at once; a thread's exponentials are added up one after the
+// other.  Measured (us, kernel by kernel, operands out of cache, one load at a time and 256 threads for every row below a
+// vocabulary / now): 8192 x 50257 bf16 606 / 574, loss alone of 4096 x 50257 249 / 162, 2048 x 4096 19.6 / 15.5, 16384 x 96 26 / 11.0.
+// (The maximum moved once for 16 values, without the order: 561, 166, 16.0 and 10.8.)
 struct MaxSum {
     float m, s;
 };
@@ -818,17 +818,16 @@ __device__ __forceinline__ MaxSum ms_merge(MaxSum a, MaxSum b) {
     const float m = fmaxf(a.m, b.m);
     return MaxSum{m, a.s * __expf(a.m - m) + b.s * __expf(b.m - m)};
 }
+// One value after the other, without a branch: x above the maximum, s exp(m - x) + 1, else s + exp(x - m).
 template <int N>
 __device__ __forceinline__ void ms_push(MaxSum &a, const float (&x)[N]) {
-    float m = a.m;
 #pragma unroll
-    for (int i = 0; i < N; i++) m = fmaxf(m, x[i]);
-    if (m > a.m) {
-        a.s *= __expf(a.m - m);
-        a.m = m;
+    for (int i = 0; i < N; i++) {
+        const bool up = x[i] > a.m;
+        const float e = __expf(-fabsf(x[i] - a.m));
+        a.s = __builtin_fmaf(up ? a.s : 1.0f, e, up ? 1.0f : a.s);
+        a.m = up ? x[i] : a.m;
     }
-#pragma unroll
-    for (int i = 0; i < N; i++) a.s += __expf(x[i] - a.m);
 }
 // Two values to 16 bits, round to nearest even, the first in the low half.
 template <int DT>
