@@ -5,7 +5,7 @@
 // of its own, the next one on its way in registers.
 //
 // Forward, the scores of a row stay in registers between the sum and P V (16 registers a block; up to NB blocks a
-// wavefront, T <= 128 NB): one walk over the keys and one exponential a score, and P is still normalised before it is narrowed.
+// wavefront, T <= 128 NB): one walk over the keys, and P is exp2(score - lse), narrowed, as in flash_kernels.hip and as the backward pass rebuilds it.
 // Backward, dQ and dK / dV are one launch; the row term, which the dQ kernel of flash_kernels.hip leaves for
 // the dK / dV kernel behind it, is formed by both.
 //
@@ -147,8 +147,6 @@ k_flash_fwd_row(const FkArgs p) {
 #pragma unroll
             for (int r = 0; r < 16; r++) e[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][r], c2, -mw));
             l += fk_sum16(e);
-#pragma unroll
-            for (int r = 0; r < 16; r++) s[t][r] = e[r];
         }
     l = fk_both(l, [](float x, float y) { return x + y; });
     st_m[L.wave][L.n] = mw;
@@ -160,7 +158,7 @@ k_flash_fwd_row(const FkArgs p) {
     l = 0.f;
 #pragma unroll
     for (int w = 0; w < 4; w++) l += st_l[w][L.n] * __builtin_amdgcn_exp2f(st_m[w][L.n] - m);
-    const float f = __builtin_amdgcn_exp2f(mw - m) / l;
+    const float lse = m + __builtin_amdgcn_logf(l);
     fk_f32x16 o[S::MB];
 #pragma unroll
     for (int i = 0; i < S::MB; i++)
@@ -175,15 +173,15 @@ k_flash_fwd_row(const FkArgs p) {
             vs.store(vt, L.lane);
             FK_WAVE_FENCE;
             if (t + 1 < NB && blk + 4 <= yb) vs.load(vb, pitch, (blk + 4) * 32, T, hd, L.lane);
-            float e[16];
+            float e[16];   // the very P that the backward pass rebuilds
 #pragma unroll
-            for (int r = 0; r < 16; r++) e[r] = s[t][r] * f;
+            for (int r = 0; r < 16; r++) e[r] = __builtin_amdgcn_exp2f(__builtin_fmaf(s[t][r], c2, -lse));
             uint32_t w[8];
             fk_narrow<DT>(e, w);
             fk_accumulate<DT, KK>(o, vt + L.trow * S::PITCH + L.tcol * 2, w);
         }
     }
-    if (L.wave == 0 && L.half == 0 && q < T) p.lse[(int64_t)blockIdx.x * T + q] = m + __builtin_amdgcn_logf(l);
+    if (L.wave == 0 && L.half == 0 && q < T) p.lse[(int64_t)blockIdx.x * T + q] = lse;
     __syncthreads();
     const int64_t row = ((int64_t)b * T + q) * D + h * hd;
     fk_meet<S::MB>(o, smem, L, [&](int d, const fk_f32x4 &v) {
