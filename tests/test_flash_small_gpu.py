@@ -51,3 +51,28 @@ def test_backward_rebuilds_the_p_of_the_forward_pass(dev, B, T, H, hd, dtype):
             b.destroy()
         forward, backward = out[:, q0:].transpose(0, 2, 1, 3), dv[:, k0:k0 + hd].transpose(0, 2, 3, 1)   # (B, H, query, key)
         assert forward.any() and np.array_equal(forward, backward)
+
+
+@pytest.mark.parametrize("T,H,hd", [(64, 256, 80), (128, 128, 96), (96, 170, 64), (64, 256, 64)])   # 510 and 512 blocks of 32 rows
+def test_backward_of_many_short_rows_is_no_slower_than_that_of_more(dev, T, H, hd):
+    """Workgroups of 32 rows took up to 512 blocks of any width and length: 28.6 us for 256 heads of 64 x 80, 21.5 for 260."""
+    from vkgrad_amd.tkernels import make_transformer_kernels
+    TK = make_transformer_kernels(dev, "bf16")
+
+    def us(H):
+        n, D = T, H * hd
+        sizes = (n * 3 * D * 2, n * D * 2, n * D * 4, 4 * H * n, 4 * H * n, n * 3 * D * 2)
+        bqkv, bg, b32, blse, bds, bdq = bufs = [dev.buffer(x, "device") for x in sizes]
+        for b in bufs:
+            b.upload(np.zeros(b.size, np.uint8))
+        g = dev.graph("backward")
+        for _ in range(8):
+            TK["flash_bwd"]([bqkv, None, bg, b32, blse, bds, bdq], 1, T, H, hd, 0.1, graph=g)
+        g.finish()
+        g.time(3)
+        t = float(np.median(g.time(15))) * 1e6 / 8
+        g.destroy()
+        for b in bufs:
+            b.destroy()
+        return t
+    assert us(H) <= 1.15 * us(H + 4)

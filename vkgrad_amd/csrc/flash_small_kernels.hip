@@ -11,8 +11,8 @@
 //
 // Bound by the chain from one block to the next, an eighth as long as with 128 rows a workgroup and all blocks in turn, against
 // four times the operand traffic from L2.
-// Measured (us, this / flash_kernels.hip): 2 heads x 1024 x 64 forward 11.4 / 28.3, backward 20.7 / 52.4; 5 x 333, 6 of 64
-// 8.6 / 14.5 and 16.7 / 27; 2 x 64, 4 of 16 3.8 / 5.0 and 5.1 / 7.9; 4 x 512, 8 of 32, packed, 8.1 / 20.3 and 15.6 / 40.7.
+// Measured (us, between others of its kind, this / flash_kernels.hip): 2 heads x 1024 x 64 forward 12.3 / 28.8, backward 21.4 / 52.4; 5 x
+// 333, 6 of 64 9.1 / 15.0 and 17.1 / 26.7; 2 x 64, 4 of 16 4.3 / 5.3 and 5.4 / 8.2; 4 x 512, 8 of 32, packed, 8.7 / 20.9 and 16.5 / 39.9.
 #include "flash_common.h"
 
 namespace mg {
@@ -367,12 +367,22 @@ k_flash_bwd_row(const FkArgs p) {
 }
 
 // The line is where four times the operand traffic costs more than idle CUs, in blocks of 32 rows.  Forward (us, here / 128 rows a
-// workgroup): 512 blocks (16 x 128, 8 of 64) 6.9 / 9.6, 696 (3 x 900, 8 of 80) 22 / 36, 1024 (8 x 512, 8 of 64) 15.4 / 19.5, 2048
-// (64 x 256, 4 of 64) 20.5 / 18.9, 2048 (4 x 1024, 16 of 64) 43 / 35.  Backward: 330 blocks 16.7 / 27, 512 16.3 / 16.0 (128 long)
-// and 15.6 / 40.7 (512 long, packed), 696 84 / 65, 1024 43 / 35.  Scores of more than 1024 keys do not fit a row's registers; the
-// tiles of four wavefronts for heads wider than 96 do not fit static LDS backward.
+// workgroup): 512 blocks (16 x 128, 8 of 64) 7.4 / 10.2, 696 (3 x 900, 8 of 80) 24 / 36, 1024 (8 x 512, 8 of 64) 16.6 / 20.2.  2048
+// (64 x 256, 4 of 64) 20.5 / 18.9, 2048 (4 x 1024, 16 of 64) 43 / 35.  Scores of more than 1024 keys do not fit a row's registers.
 bool fk_small_forward(const FkArgs &a, int64_t nbh) { return a.T <= 1024 && nbh * ((a.T + 31) / 32) <= 1024; }
-bool fk_small_backward(const FkArgs &a, int64_t nbh) { return fk_steps(a.hd) <= 6 && nbh * ((a.T + 31) / 32) <= 512; }
+// Backward a block is two workgroups, of which a CU holds two with heads of up to 64 and one with wider ones (324 registers): the
+// rounds are 256 and 128 blocks, and as many of them are worth it as a row is long, whose chain they shorten.  Heads of 32: 512
+// blocks of 64 rows 9.8 / 9.3, of 256 14 / 18.  Heads of 64: 256 blocks of 64 rows 9 / 11, 320 13 / 11; 384 of 128 16 / 16.6, 512 17.4 / 17; 384 of 160
+// 16 / 18, 512 20 / 19; 512 of 256 21 / 23.  Heads of 80: 128 blocks of 64 rows 9 / 12.5, 256 15 / 13.5; 256 of 128 16 / 19, 320 21 / 19; 320
+// of 256 25 / 27, 448 33 / 28; 384 of 512 34 / 40, 512 45 / 42.  The tiles of four wavefronts for heads wider than 96 do not fit static LDS.
+bool fk_small_backward(const FkArgs &a, int64_t nbh) {
+    const int steps = fk_steps(a.hd);
+    const int most = steps <= 2 ? 512
+                     : steps == 4 ? (a.T < 128 ? 256 : a.T < 256 ? 384 : 512)
+                     : steps == 6 ? (a.T < 128 ? 128 : a.T < 256 ? 256 : a.T < 512 ? 320 : 384)
+                                  : 0;
+    return nbh * ((a.T + 31) / 32) <= most;
+}
 
 template <int DT, int KK>
 static void fk_small_forward_launch(hipStream_t s, const FkArgs &a, dim3 grid) {
