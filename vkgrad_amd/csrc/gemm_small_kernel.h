@@ -1,9 +1,9 @@
 // Products that take microseconds: the plan of the 64 x 64 tile - its K slices, and the order in which each adds up - run with
 // a wavefront a slice instead of a workgroup a slice.
 //
-// A workgroup owns 32 x 32 outputs; wavefront s takes K slice s, asks for all of its operands at once (up to four K-blocks of
-// 64) and multiplies them without meeting anybody: K-contiguous operands go from memory straight into MFMA
-// fragments, the N-contiguous B of layout NN through a few kilobytes of LDS of the wavefront's own, read back transposed.
+// A workgroup owns 32 x 32 outputs; wavefront s takes K slice s, asks for the operands of four K-blocks of 64 at once (two where B comes
+// element by element; the rule that takes a product keeps most slices to that) and multiplies them without meeting anybody:
+// K-contiguous operands go from memory straight into MFMA fragments, the N-contiguous B of layout NN through a few kilobytes of LDS of the wavefront's own, read back transposed.
 // The partial sums meet in LDS, added in slice order, and one wavefront runs the usual epilogue: the bits are those of the
 // slices that meet in the workspace, without its round trip through memory, its counter and its waiting.
 //
