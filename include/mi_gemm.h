@@ -235,11 +235,16 @@ int mg_gemm(mg_ctx *ctx, const mg_gemm_args *args);
 /* The backward pass of a linear layer (autograd.py:213-228, transformer.py:97-109: two Matmul calls
  * and a column sum): dw, then db, then dx, as mg_gemm and mg_ew_col_sum / mg_tk_col_sum16 give
  * them - in one launch where that is estimated to be faster, the three of them
- * side by side on the chip. */
+ * side by side on the chip.  A tile or a K split that dw or dx names (tile >= 0, split_k > 0) is what that product runs with, in
+ * one launch as in several: with MG_BACKWARD_AUTO the one launch is considered with no other, and there is none for most tiles.
+ * With MG_BACKWARD_REPLAN the one launch has its own tile and K slices whatever the products name, and is compared with what they
+ * name: for plans that were measured on a product by itself.  Other K slices add up in another order: results agree with the
+ * launches in turn up to the rounding of f32 sums, and exactly where tile and slices are the same.  MG_FLAG_SPLITK_SUM changes
+ * no bits, and nothing here. */
 typedef struct mg_backward_args {
     int32_t struct_size;           /* sizeof(mg_backward_args) */
-    int32_t tile;                  /* MG_BACKWARD_AUTO: one launch or several, by estimate; MG_BACKWARD_APART: several, each as
-                                      mg_gemm runs it; a tile id: one launch with that tile (MG_ERR_ARG where there is none) */
+    int32_t tile;                  /* MG_BACKWARD_AUTO, MG_BACKWARD_REPLAN: one launch or several, by estimate; MG_BACKWARD_APART: several,
+                                      each as mg_gemm runs it; a tile id: one launch with that tile (MG_ERR_ARG where there is none) */
     int32_t split_w, split_x;      /* K slices of the products with a named tile (0: one) */
     const mg_gemm_args *dw;        /* layout TN, one batch */
     const mg_gemm_args *dx;        /* layout NT or NN, one batch, the type of dw; NULL: not wanted */
@@ -250,6 +255,7 @@ typedef struct mg_backward_args {
 } mg_backward_args;
 #define MG_BACKWARD_AUTO (-1)
 #define MG_BACKWARD_APART (-2)
+#define MG_BACKWARD_REPLAN (-3)
 int mg_gemm_backward(mg_ctx *ctx, const mg_backward_args *args);
 /* What it runs on a device with `compute_units` CUs: the tile and the K slices of the one launch, or
  * MG_BACKWARD_APART; pure arithmetic. */

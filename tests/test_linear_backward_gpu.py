@@ -122,3 +122,60 @@ def test_refused_where_it_is_recorded(which):
     with pytest.raises(VkError):
         record()
     assert g.n_dispatch == 1
+
+
+def test_named_plans_bind():
+    """A tile or K split that a product names is what it runs with, in one launch or by itself; MG_BACKWARD_REPLAN is for plans that
+    were measured on a product by itself."""
+    lib = L.load()
+
+    def pick(rows, fin, fout, how=L.MG_BACKWARD_AUTO, w=(-1, 0), x=(-1, 0)):
+        bufs = {n: _Mem((i + 1) << 33) for i, n in enumerate(("x", "w", "dy", "dw", "dx", "y", "z", "g32", "db"))}
+        b = _args(bufs, rows, fin, fout, how, 0, 0, "bf16", "plain", "16", False)
+        (b.dw.contents.tile, b.dw.contents.split_k), (b.dx.contents.tile, b.dx.contents.split_k) = w, x
+        out = [C.c_int() for _ in range(3)]
+        assert lib.mg_backward_pick(C.byref(b), 256, *(C.byref(o) for o in out)) == L.MG_OK
+        return tuple(o.value for o in out)
+
+    apart = (L.MG_BACKWARD_APART, 0, 0)
+    for shape, w in (((8192, 768, 3072), (21, 5)), ((1665, 384, 1152), (11, 1)), ((128, 64, 256), (3, 2)), ((4096, 1024, 1024), (11, 3))):
+        free, bound = pick(*shape), pick(*shape, w=w)
+        assert free[0] >= 0 and free[:2] != w
+        assert bound == apart or bound[:2] == w
+        assert pick(*shape, how=L.MG_BACKWARD_REPLAN, w=w)[0] >= 0     # (compared with what the named plan takes)
+    assert pick(128, 64, 256, w=(3, 2)) == apart                       # no one-launch kernel has that tile
+    assert pick(1665, 384, 1152, w=(4, 2), x=(4, 1)) == (4, 2, 1)
+    assert pick(1665, 384, 1152, w=(4, 1), x=(11, 1)) == apart
+    assert pick(1665, 384, 1152, x=(-1, 2))[2] in (0, 2) and pick(1665, 384, 1152, w=(-1, 2))[1] in (0, 2)
+    assert pick(8192, 768, 3072, x=(21, 2)) == apart
+
+
+def test_whose_plans_bind(monkeypatch):
+    """Plans from the shipped table give way to the one launch, plans that the caller or the tuner named do not."""
+    from vkgrad_amd import kernels as K
+    from vkgrad_amd.autograd import Ctx
+
+    class Dev:
+        _lib, _ctx, name, compute_units = L.load(), None, "fake", 256
+
+    entry = {"tile_id": 11, "split_k": 3, "group_m": 4}
+    key = K.tune_key("fake", 64, 64, 32, True, False)
+    bufs = {n: _Mem((i + 1) << 33) for i, n in enumerate(("x", "w", "dy", "dw", "dx"))}
+
+    def recorded(mw, mx):
+        g = Graph(Dev(), "g")
+        linear_backward(Dev(), (mw, (bufs["x"], bufs["dy"], bufs["dw"], 64, 64, 32), {}),
+                        (mx, (bufs["dy"], bufs["w"], bufs["dx"], 32, 64, 64), {}), graph=g)
+        return g._thunks[0].__defaults__[0].tile
+
+    plain = Matmul(Dev(), trans_b=True)
+    assert recorded(Matmul(Dev(), trans_a=True), plain) == L.MG_BACKWARD_AUTO
+    assert recorded(Matmul(Dev(), trans_a=True, tile=11), plain) == L.MG_BACKWARD_AUTO
+    for shipped, user, want in (({key: entry}, {}, L.MG_BACKWARD_REPLAN), ({}, {key: entry}, L.MG_BACKWARD_AUTO)):
+        monkeypatch.setattr(K, "_shipped_table", lambda t=shipped: t)
+        monkeypatch.setattr(K, "_load_cache", lambda path=None, t=user: t)
+        ctx = Ctx.__new__(Ctx)
+        ctx.dev, ctx.tune, ctx.dtype, ctx._mm = Dev(), False, "f16", {}
+        mm = ctx.matmul(64, 64, 32, trans_a=True)
+        assert mm.tile == 11 and recorded(mm, plain) == want
+        assert recorded(mm, Matmul(Dev(), trans_b=True, split_k=2)) == L.MG_BACKWARD_AUTO

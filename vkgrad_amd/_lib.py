@@ -23,7 +23,7 @@ MG_COPY_MAX = 8
 
 DTYPES = {"f16": MG_F16, "bf16": MG_BF16}
 KINDS = {"device": MG_DEVICE, "shared": MG_SHARED, "cached": MG_CACHED, "bar": MG_BAR}
-MG_BACKWARD_AUTO, MG_BACKWARD_APART = -1, -2
+MG_BACKWARD_AUTO, MG_BACKWARD_APART, MG_BACKWARD_REPLAN = -1, -2, -3
 MG_ACT_GELU_GRAD, MG_ACT_RELU_GRAD, MG_ACT_SOFTMAX_GRAD = 3, 4, 5
 TRI = {None: 0, "c_lower": 1, "a_lower": 2, "a_upper": 3}
 ACTS = {None: MG_ACT_NONE, "none": MG_ACT_NONE, "gelu": MG_ACT_GELU, "relu": MG_ACT_RELU,

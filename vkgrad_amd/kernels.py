@@ -96,6 +96,8 @@ class Matmul:
                      f"{'_bat' if batched else ''}{'_g' + str(group_m) if group_m else ''}"
                      f"{'_s' + str(split_k) if split_k > 1 else ''}{'_at' if atomic_split else ''}"
                      f"{'' if xcd_rotate is None else ('_rot' if xcd_rotate else '_ins')}")
+        # the plan is the shipped table's, measured on the product by itself: `linear_backward` may take another
+        self.from_table = False
         self._keep = []
         self._sent = {}   # enqueue's checked arguments
 
@@ -338,7 +340,8 @@ def linear_backward(dev, dw, dx=None, db=None, graph=None):
     """The backward pass of a linear layer: dW, the bias gradient and dX, which share no result, in one
     launch where the library estimates that to be faster (autograd.py:213-228 issues them in turn).
     dw, dx: (Matmul, positional arguments, keyword arguments) of its call; db: (matrix, sums,
-    columns, rows, accumulate, f32) - the column sums of a dense matrix, f32 or 16 bits."""
+    columns, rows, accumulate, f32) - the column sums of a dense matrix, f32 or 16 bits.  A tile or a K split
+    that a Matmul was made with is what its product runs with, except from the shipped table (`from_table`)."""
     lib, ctx = dev._lib, dev._ctx
     args, buffers, traffic, splits = [], [], 0, []
     for mm, (a, b, c, m, n, k), kw in (p for p in (dw, dx) if p is not None):
@@ -352,6 +355,9 @@ def linear_backward(dev, dw, dx=None, db=None, graph=None):
         splits.append((2 * (m * k + k * n), m * n * 4))
     ba = L.BackwardArgs()
     ba.struct_size, ba.tile = C.sizeof(L.BackwardArgs), L.MG_BACKWARD_AUTO
+    named = [p[0] for p in (dw, dx) if p is not None and (p[0].tile >= 0 or p[0].split_k > 0)]
+    if named and all(mm.from_table for mm in named):
+        ba.tile = L.MG_BACKWARD_REPLAN
     ba.dw = C.pointer(args[0])   # (ctypes keeps what a pointer points to)
     if dx is not None:
         ba.dx = C.pointer(args[1])
@@ -495,6 +501,11 @@ def lookup_tuned(dev_name, m, n, k, trans_a, trans_b, dtype="f16", batched=False
             if e is not None:
                 return e
     return None
+
+
+def is_shipped(e):
+    """Whether lookup_tuned found the entry in the shipped table, not in the user's cache."""
+    return any(e is x for x in _shipped_table().values())
 
 
 def matmul_from_entry(dev, e, trans_a=False, trans_b=False, dtype="f16", batched=False):
