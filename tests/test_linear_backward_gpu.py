@@ -179,3 +179,31 @@ def test_whose_plans_bind(monkeypatch):
         mm = ctx.matmul(64, 64, 32, trans_a=True)
         assert mm.tile == 11 and recorded(mm, plain) == want
         assert recorded(mm, Matmul(Dev(), trans_b=True, split_k=2)) == L.MG_BACKWARD_AUTO
+
+
+def test_keywords_of_a_product_arrive():
+    """Every keyword of Matmul's call reaches the product, with its buffer; others are refused."""
+    class Dev:
+        _lib, _ctx = L.load(), None
+
+    bufs = {n: _Mem((i + 1) << 33) for i, n in enumerate(("x", "w", "dy", "dw", "dx", "res", "bias"))}
+
+    def record(graph=True, **kw):
+        g = Graph(Dev(), "g") if graph else None
+        linear_backward(Dev(), (Matmul(Dev(), trans_a=True), (bufs["x"], bufs["dy"], bufs["dw"], 64, 64, 32), dict(ldc=72, accumulate=True)),
+                        (Matmul(Dev(), trans_b=True), (bufs["dy"], bufs["w"], bufs["dx"], 32, 64, 64), kw), graph=g)
+        return g
+
+    g = record(res=bufs["res"], ldr=80, bias=bufs["bias"], lda=96, ldb=104, ldc=112)
+    ba = g._thunks[0].__defaults__[0]
+    dw, dx = ba.dw.contents, ba.dx.contents
+    assert (dw.lda, dw.ldb, dw.ldc, dw.beta) == (64, 64, 72, 1)
+    assert (dx.lda, dx.ldb, dx.ldc, dx.beta, dx.res, dx.ldr, dx.bias) == (96, 104, 112, 1, bufs["res"].ptr, 80, bufs["bias"].ptr)
+    assert all(id(b) in g._buffers for b in bufs.values())
+    assert record(side=True)._thunks[0].__defaults__[0].dx.contents.flags & L.MG_FLAG_SIDE_STREAM
+    with pytest.raises(VkError):
+        record(graph=False, side=True)
+    with pytest.raises(TypeError):
+        record(acumulate=True)
+    with pytest.raises(VkError):
+        record(tri="diagonal")

@@ -345,12 +345,14 @@ def linear_backward(dev, dw, dx=None, db=None, graph=None):
     lib, ctx = dev._lib, dev._ctx
     args, buffers, traffic, splits = [], [], 0, []
     for mm, (a, b, c, m, n, k), kw in (p for p in (dw, dx) if p is not None):
-        get = kw.get
-        args.append(mm._args(a, b, c, m, n, k, 1, (0, 0, 0), get("bias"), get("accumulate", False), None, None, None,
-                             act=get("act"), y16=get("y16"), z=get("z"), colsum=get("colsum")))
+        if kw.get("side") and graph is None:
+            raise VkError(f"{mm.name}: side=True needs graph=")
+        named = dict(bias=None, accumulate=False, lda=None, ldb=None, ldc=None)
+        named.update(kw)   # (what a product does not take is refused by name)
+        args.append(mm._args(a, b, c, m, n, k, 1, (0, 0, 0), **named))
         if graph is not None:   # refused where it is recorded, like a product by itself
             _check(lib.mg_gemm_check(C.byref(args[-1])), mm.name)
-        buffers += [x for x in (a, b, c, *(get(x) for x in ("bias", "y16", "z", "colsum"))) if x is not None]
+        buffers += [x for x in (a, b, c, *kw.values()) if hasattr(x, "ptr")]
         traffic += mm.traffic_bytes(m, n, k)
         splits.append((2 * (m * k + k * n), m * n * 4))
     ba = L.BackwardArgs()
