@@ -77,9 +77,7 @@ __global__ void k_act_bwd(const float *dy, const float *z, uint16_t *dz16, float
 // row pieces), LDS adds the 8 partial sums.  One chunk of rows: the block writes (or adds to) the
 // sum itself, in a fixed order.  More rows: the chunks add with atomics into sums, which the
 // host has cleared unless accumulating.
-constexpr int COL_SUM_ROWS = 512;
 // Up to COL_SUM_ONE rows one chunk with twice the threads per column takes them all: no clear in front, no atomics.
-constexpr int COL_SUM_ONE = 1024;
 // 16 columns a workgroup: with 64, 2049 columns kept 33 CUs busy with 256 KB each (1000 rows 10.5 us, 8.1 so).  Rows beyond the
 // end are clamped and not added: what an unrolled loop leaves over would be loaded one by one.
 constexpr int COL_SUM_ONE_COLS = 16;

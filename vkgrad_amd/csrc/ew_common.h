@@ -27,6 +27,21 @@ __device__ __forceinline__ float widen16(uint16_t h, int dtype) {
     return __builtin_bit_cast(float, (uint32_t)h << 16);
 }
 
+// Two values to 16 bits, round to nearest even, the first in the low half.
+template <int DT>
+__device__ __forceinline__ uint32_t pack16(float a, float b) {
+    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    if constexpr (DT == MG_F16) return __builtin_bit_cast(uint32_t, h2{(_Float16)a, (_Float16)b});
+    else return __builtin_bit_cast(uint32_t, b2{(__bf16)a, (__bf16)b});
+}
+
+// Column sums: rows of a chunk - several chunks add with atomics -, and how many rows of an f32 matrix one chunk of
+// twice the threads takes at the most.  The sums that share a launch with products (gemm_backward_kernel.h) have the same chunks, and so
+// the same bits.
+constexpr int COL_SUM_ROWS = 512;
+constexpr int COL_SUM_ONE = 1024;
+
 static inline unsigned blocks_for(int64_t n) { return (unsigned)((n + 255) / 256); }
 static inline bool dtype_ok(int d) { return d == MG_F16 || d == MG_BF16; }
 static inline bool count_ok(int64_t n) { return n > 0 && n <= (int64_t)0x7fffffff * 256; }

@@ -12,8 +12,6 @@ namespace mg {
 
 typedef _Float16 fk_half8 __attribute__((ext_vector_type(8)));
 typedef __bf16 fk_bf8 __attribute__((ext_vector_type(8)));
-typedef _Float16 fk_half2 __attribute__((ext_vector_type(2)));
-typedef __bf16 fk_bf2 __attribute__((ext_vector_type(2)));
 typedef float fk_f32x16 __attribute__((ext_vector_type(16)));
 typedef float fk_f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t fk_u32x4 __attribute__((ext_vector_type(4)));
@@ -27,12 +25,6 @@ __device__ __forceinline__ fk_f32x16 fk_mfma(fk_u32x4 a, fk_u32x4 b, fk_f32x16 c
         return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(fk_half8, a), __builtin_bit_cast(fk_half8, b), c, 0, 0, 0);
     else
         return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(fk_bf8, a), __builtin_bit_cast(fk_bf8, b), c, 0, 0, 0);
-}
-// Two values to 16 bits, round to nearest even, the first in the low half.
-template <int DT>
-__device__ __forceinline__ uint32_t fk_pack(float a, float b) {
-    if constexpr (DT == MG_F16) return __builtin_bit_cast(uint32_t, fk_half2{(_Float16)a, (_Float16)b});
-    else return __builtin_bit_cast(uint32_t, fk_bf2{(__bf16)a, (__bf16)b});
 }
 template <int DT>
 __device__ __forceinline__ float fk_widen(uint32_t b) {
@@ -51,7 +43,7 @@ template <int DT>
 __device__ __forceinline__ void fk_round(float (&e)[16], uint32_t (&w)[8]) {
 #pragma unroll
     for (int r = 0; r < 16; r += 2) {
-        const uint32_t u = fk_pack<DT>(e[r], e[r + 1]);
+        const uint32_t u = pack16<DT>(e[r], e[r + 1]);
         w[r / 2] = u;
         e[r] = fk_widen<DT>(u & 0xffffu);
         e[r + 1] = fk_widen<DT>(u >> 16);
@@ -60,7 +52,7 @@ __device__ __forceinline__ void fk_round(float (&e)[16], uint32_t (&w)[8]) {
 template <int DT>
 __device__ __forceinline__ void fk_narrow(const float (&e)[16], uint32_t (&w)[8]) {
 #pragma unroll
-    for (int r = 0; r < 16; r += 2) w[r / 2] = fk_pack<DT>(e[r], e[r + 1]);
+    for (int r = 0; r < 16; r += 2) w[r / 2] = pack16<DT>(e[r], e[r + 1]);
 }
 
 constexpr int FK_BN = 64;   // rows of a staged tile
@@ -150,8 +142,8 @@ __device__ __forceinline__ void fk_store_row16(uint16_t *row, const fk_f32x16 (&
         for (int g = 0; g < 4; g++) {
             const int d = 32 * i + 8 * g + 4 * half;
             if (d < hd)
-                *reinterpret_cast<fk_u32x2 *>(row + d) = fk_u32x2{fk_pack<DT>(o[i][4 * g] * f, o[i][4 * g + 1] * f),
-                                                                  fk_pack<DT>(o[i][4 * g + 2] * f, o[i][4 * g + 3] * f)};
+                *reinterpret_cast<fk_u32x2 *>(row + d) = fk_u32x2{pack16<DT>(o[i][4 * g] * f, o[i][4 * g + 1] * f),
+                                                                  pack16<DT>(o[i][4 * g + 2] * f, o[i][4 * g + 3] * f)};
         }
 }
 
@@ -173,6 +165,25 @@ __device__ __forceinline__ float fk_sum16(const float (&v)[16]) {
 #pragma unroll
     for (int i = 0; i < 4; i++) t[i] = (v[i] + v[4 + i]) + (v[8 + i] + v[12 + i]);
     return (t[0] + t[1]) + (t[2] + t[3]);
+}
+
+// sum over d of g16[d] out32[d] for this lane's row, its half of the columns; both halves hold the sum
+template <int DT, int KK>
+__device__ __forceinline__ float fk_row_term(const fk_u32x4 (&g)[KK], const float *row, int half, int hd) {
+    float t = 0.f;
+#pragma unroll
+    for (int kk = 0; kk < KK; kk++) {
+        const int d = kk * 16 + half * 8;
+        if (d < hd) {
+            const fk_f32x4 x = *reinterpret_cast<const fk_f32x4 *>(row + d), y = *reinterpret_cast<const fk_f32x4 *>(row + d + 4);
+#pragma unroll
+            for (int w = 0; w < 4; w++) {
+                const float lo = fk_widen<DT>(g[kk][w] & 0xffffu), hi = fk_widen<DT>(g[kk][w] >> 16);
+                t += w < 2 ? lo * x[2 * w] + hi * x[2 * w + 1] : lo * y[2 * w - 4] + hi * y[2 * w - 3];
+            }
+        }
+    }
+    return fk_both(t, [](float a, float b) { return a + b; });
 }
 
 // Where the lanes of a wavefront read a tile: block b's rows as A operands, and transposed.

@@ -194,21 +194,7 @@ k_flash_dq(const FkArgs p) {
     fk_u32x4 qf[KK], gf[KK];
     fk_load_row<KK>(qf, qb + qc * pitch, L.half, hd);
     fk_load_row<KK>(gf, p.dout + orow, L.half, hd);
-    float dsum = 0.f;
-#pragma unroll
-    for (int kk = 0; kk < KK; kk++) {
-        const int d = kk * 16 + L.half * 8;
-        if (d < hd) {
-            const fk_f32x4 x = *reinterpret_cast<const fk_f32x4 *>(p.out32 + orow + d);
-            const fk_f32x4 y = *reinterpret_cast<const fk_f32x4 *>(p.out32 + orow + d + 4);
-#pragma unroll
-            for (int w = 0; w < 4; w++) {
-                const float lo = fk_widen<DT>(gf[kk][w] & 0xffffu), hi = fk_widen<DT>(gf[kk][w] >> 16);
-                dsum += w < 2 ? lo * x[2 * w] + hi * x[2 * w + 1] : lo * y[2 * w - 4] + hi * y[2 * w - 3];
-            }
-        }
-    }
-    dsum += __shfl_xor(dsum, 32, 64);
+    const float dsum = fk_row_term<DT, KK>(gf, p.out32 + orow, L.half, hd);
     const int64_t stat = (int64_t)wk.bh * T + qc;
     if (L.half == 0 && q < T) p.dsum[stat] = dsum;
     const float lse = p.lse[stat], dscaled = dsum * p.scale;

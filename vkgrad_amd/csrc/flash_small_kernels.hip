@@ -80,7 +80,7 @@ __device__ __forceinline__ void fk_meet(const fk_f32x16 (&o)[MB], char *lds, con
 }
 template <int DT>
 __device__ __forceinline__ void fk_put16(uint16_t *row, int d, const fk_f32x4 &v, int hd) {
-    if (d < hd) *reinterpret_cast<fk_u32x2 *>(row + d) = fk_u32x2{fk_pack<DT>(v[0], v[1]), fk_pack<DT>(v[2], v[3])};
+    if (d < hd) *reinterpret_cast<fk_u32x2 *>(row + d) = fk_u32x2{pack16<DT>(v[0], v[1]), pack16<DT>(v[2], v[3])};
 }
 __device__ __forceinline__ int fk_first_block(int first) {
     int f = first;
@@ -189,25 +189,6 @@ k_flash_fwd_row(const FkArgs p) {
         fk_put16<DT>(p.out16 + row, d, v, hd);
         if (p.out32) *reinterpret_cast<fk_f32x4 *>(p.out32 + row + d) = v;
     });
-}
-
-// sum over d of g16[d] out32[d] for this lane's row, its half of the columns; both halves hold the sum
-template <int DT, int KK>
-__device__ __forceinline__ float fk_row_term(const fk_u32x4 (&g)[KK], const float *row, int half, int hd) {
-    float t = 0.f;
-#pragma unroll
-    for (int kk = 0; kk < KK; kk++) {
-        const int d = kk * 16 + half * 8;
-        if (d < hd) {
-            const fk_f32x4 x = *reinterpret_cast<const fk_f32x4 *>(row + d), y = *reinterpret_cast<const fk_f32x4 *>(row + d + 4);
-#pragma unroll
-            for (int w = 0; w < 4; w++) {
-                const float lo = fk_widen<DT>(g[kk][w] & 0xffffu), hi = fk_widen<DT>(g[kk][w] >> 16);
-                t += w < 2 ? lo * x[2 * w] + hi * x[2 * w + 1] : lo * y[2 * w - 4] + hi * y[2 * w - 3];
-            }
-        }
-    }
-    return fk_both(t, [](float a, float b) { return a + b; });
 }
 
 // ---- backward ------------------------------------------------------------------------

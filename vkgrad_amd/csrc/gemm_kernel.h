@@ -21,6 +21,7 @@
 #include <stdint.h>
 
 #include "act_math.h"
+#include "ew_common.h"
 
 namespace mg {
 
@@ -591,16 +592,6 @@ __device__ __forceinline__ void store_tile(const GemmParams &p, float *C, f32x16
 // GEMM).  Here each wavefront turns 32 rows of its tile at a time through LDS of its own (the ring is done by
 // then) and every lane takes eight neighbouring columns of a row: one 16-byte store of Y, two of C, two loads
 // of Z, R or C.  The pitch of WTN + 8 floats puts the two half-waves' rows on different banks.
-template <int DT>
-__device__ __forceinline__ uint32_t pack16(float a, float b) {
-    if constexpr (DT == D_F16) {
-        typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-        return __builtin_bit_cast(uint32_t, h2{(_Float16)a, (_Float16)b});
-    } else {
-        typedef __bf16 b2 __attribute__((ext_vector_type(2)));
-        return __builtin_bit_cast(uint32_t, b2{(__bf16)a, (__bf16)b});
-    }
-}
 // ACTV: MG_ACT_*, known at compile time - a test of it per element would put every exponential in a basic block
 // of its own, one dependent chain after the other.
 template <int DT, int TM, int TN, int WTM, int WTN, int NW, int ACTV>

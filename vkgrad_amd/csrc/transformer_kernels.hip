@@ -762,7 +762,6 @@ __global__ void k_add_bias(float *x, const float *bias, int64_t n, int64_t ncol)
 // 8 columns and 256 rows per block: 6.7 us against 5.3 - 6.2 us for 8192 x 768, no gain.)
 // Two matrices of one shape share a launch (grid.z), the gradients of a norm's gain and shift: 2048 x 512 5.3 us each apart,
 // 5.3 for both.
-constexpr int CS16_ROWS = 512;
 struct ColSum16 {
     const uint16_t *g[2];
     float *sums[2];
@@ -774,8 +773,8 @@ k_col_sum16(const ColSum16 a, int64_t ncol, int64_t nrow, int accumulate, int at
     const uint16_t *g = a.g[blockIdx.z];
     float *sums = a.sums[blockIdx.z];
     const int64_t c = (int64_t)blockIdx.x * 64 + tx;
-    const int64_t r0 = (int64_t)blockIdx.y * CS16_ROWS;
-    const int64_t r1 = r0 + CS16_ROWS < nrow ? r0 + CS16_ROWS : nrow;
+    const int64_t r0 = (int64_t)blockIdx.y * COL_SUM_ROWS;
+    const int64_t r1 = r0 + COL_SUM_ROWS < nrow ? r0 + COL_SUM_ROWS : nrow;
     float s = 0.f;
     if (c < ncol) {
 #pragma unroll 8
@@ -828,14 +827,6 @@ __device__ __forceinline__ void ms_push(MaxSum &a, const float (&x)[N]) {
         a.s = __builtin_fmaf(up ? a.s : 1.0f, e, up ? 1.0f : a.s);
         a.m = up ? x[i] : a.m;
     }
-}
-// Two values to 16 bits, round to nearest even, the first in the low half.
-template <int DT>
-__device__ __forceinline__ uint32_t ce_pack(float a, float b) {
-    typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
-    if constexpr (DT == MG_F16) return __builtin_bit_cast(uint32_t, h2{(_Float16)a, (_Float16)b});
-    else return __builtin_bit_cast(uint32_t, b2{(__bf16)a, (__bf16)b});
 }
 constexpr int CE_ILP = 4;
 template <int NT, int DT>
@@ -916,7 +907,7 @@ k_softmax_ce_wide(const float *logits, const uint32_t *labels, const float *weig
             d -= e == 3 ? 1.f : 0.f;
         }
         a *= w; b *= w; cc *= w; d *= w;
-        if (g16) reinterpret_cast<uint2 *>(g16)[c] = make_uint2(ce_pack<DT>(a, b), ce_pack<DT>(cc, d));
+        if (g16) reinterpret_cast<uint2 *>(g16)[c] = make_uint2(pack16<DT>(a, b), pack16<DT>(cc, d));
         if (g32) reinterpret_cast<float4 *>(g32)[c] = make_float4(a, b, cc, d);
     };
     for (c = tid; c + (CE_ILP - 1) * NT < n4; c += CE_ILP * NT) {
@@ -1174,7 +1165,7 @@ int mg_tk_add_bias(mg_ctx *ctx, float *x, const float *bias, int64_t n, int64_t 
 }
 
 static int col_sum16(mg_ctx *ctx, const ColSum16 &a, int n, int64_t ncol, int64_t nrow, int accumulate, int dtype, const char *name) {
-    const unsigned chunks = (unsigned)((nrow + CS16_ROWS - 1) / CS16_ROWS);
+    const unsigned chunks = (unsigned)((nrow + COL_SUM_ROWS - 1) / COL_SUM_ROWS);
     if (chunks > 1 && !accumulate)
         for (int i = 0; i < n; i++) hipLaunchKernelGGL(k_zero_f32, dim3(blocks_for(ncol)), dim3(256), 0, ctx_stream(ctx), a.sums[i], ncol);
     hipLaunchKernelGGL(k_col_sum16, dim3((unsigned)((ncol + 63) / 64), chunks, (unsigned)n), dim3(512), 0, ctx_stream(ctx), a, ncol, nrow,
@@ -1183,7 +1174,7 @@ static int col_sum16(mg_ctx *ctx, const ColSum16 &a, int n, int64_t ncol, int64_
 }
 
 int mg_tk_col_sum16(mg_ctx *ctx, const void *g16, float *sums, int64_t ncol, int64_t nrow, int accumulate, int dtype) {
-    EW_PRECHECK("mg_tk_col_sum16", g16 && sums && count_ok(ncol) && nrow > 0 && nrow <= (int64_t)65535 * CS16_ROWS &&
+    EW_PRECHECK("mg_tk_col_sum16", g16 && sums && count_ok(ncol) && nrow > 0 && nrow <= (int64_t)65535 * COL_SUM_ROWS &&
                                        dtype_ok(dtype));
     return col_sum16(ctx, ColSum16{{(const uint16_t *)g16, nullptr}, {sums, nullptr}}, 1, ncol, nrow, accumulate, dtype, "mg_tk_col_sum16");
 }
@@ -1191,7 +1182,7 @@ int mg_tk_col_sum16(mg_ctx *ctx, const void *g16, float *sums, int64_t ncol, int
 int mg_tk_col_sum16_pair(mg_ctx *ctx, const void *a16, float *a_sums, const void *b16, float *b_sums, int64_t ncol, int64_t nrow,
                          int accumulate, int dtype) {
     EW_PRECHECK("mg_tk_col_sum16_pair", a16 && a_sums && b16 && b_sums && a_sums != b_sums && count_ok(ncol) && nrow > 0 &&
-                                            nrow <= (int64_t)65535 * CS16_ROWS && dtype_ok(dtype));
+                                            nrow <= (int64_t)65535 * COL_SUM_ROWS && dtype_ok(dtype));
     return col_sum16(ctx, ColSum16{{(const uint16_t *)a16, (const uint16_t *)b16}, {a_sums, b_sums}}, 2, ncol, nrow, accumulate, dtype,
                      "mg_tk_col_sum16_pair");
 }
