@@ -352,17 +352,22 @@ k_flash_bwd_row(const FkArgs p) {
 // (64 x 256, 4 of 64) 20.5 / 18.9, 2048 (4 x 1024, 16 of 64) 43 / 35.  Scores of more than 1024 keys do not fit a row's registers.
 bool fk_small_forward(const FkArgs &a, int64_t nbh) { return a.T <= 1024 && nbh * ((a.T + 31) / 32) <= 1024; }
 // Backward a block is two workgroups, of which a CU holds two with heads of up to 64 and one with wider ones (324 registers): the
-// rounds are 256 and 128 blocks, and as many of them are worth it as a row is long, whose chain they shorten.  Heads of 32: 512
-// blocks of 64 rows 9.8 / 9.3, of 256 14 / 18.  Heads of 64: 256 blocks of 64 rows 9 / 11, 320 13 / 11; 384 of 128 16 / 16.6, 512 17.4 / 17; 384 of 160
-// 16 / 18, 512 20 / 19; 512 of 256 21 / 23.  Heads of 80: 128 blocks of 64 rows 9 / 12.5, 256 15 / 13.5; 256 of 128 16 / 19, 320 21 / 19; 320
-// of 256 25 / 27, 448 33 / 28; 384 of 512 34 / 40, 512 45 / 42.  The tiles of four wavefronts for heads wider than 96 do not fit static LDS.
+// rounds are 256 and 128 blocks, and more of them are worth it the longer a row is, whose chain they shorten, and in packed rows, where
+// 128 rows walk the tiles of the earliest of them.  Where 128 rows a workgroup overtake (their time over this one's; 32 to 1024 rows,
+// 128 to 512 blocks, bf16): heads of 32 nowhere (512 blocks of 64 rows 0.95, of 256 1.28); of 64, 64 rows 256 blocks 1.19, 320 0.90, 96 rows
+// 312 1.09, 384 0.96 (packed 504 1.02), 128 rows 512 0.99; of 80, 64 rows 128 blocks 1.39, 192 0.89, 128 rows 256 1.18, 320 0.92 (packed
+// 1.03), 256 rows 320 1.08, 384 0.99, 448 0.84 (packed 1.04), 512 rows 384 1.17, 448 0.97, packed 512 1.14.  The tiles of four wavefronts for heads
+// wider than 96 do not fit static LDS.
+static int fk_small_backward_most(int steps, int T, bool packed) {
+    if (steps <= 2) return 512;
+    if (steps == 4) return T <= 64 ? 256 : T < 128 && !packed ? 320 : 512;
+    if (steps > 6) return 0;
+    if (T < 96) return 128;
+    if (T < 256) return packed && T >= 128 ? 320 : 256;
+    return T < 384 ? (packed ? 448 : 320) : packed ? 512 : 384;
+}
 bool fk_small_backward(const FkArgs &a, int64_t nbh) {
-    const int steps = fk_steps(a.hd);
-    const int most = steps <= 2 ? 512
-                     : steps == 4 ? (a.T < 128 ? 256 : a.T < 256 ? 384 : 512)
-                     : steps == 6 ? (a.T < 128 ? 128 : a.T < 256 ? 256 : a.T < 512 ? 320 : 384)
-                                  : 0;
-    return nbh * ((a.T + 31) / 32) <= most;
+    return nbh * ((a.T + 31) / 32) <= fk_small_backward_most(fk_steps(a.hd), a.T, a.seg != nullptr);
 }
 
 template <int DT, int KK>
