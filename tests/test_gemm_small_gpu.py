@@ -39,15 +39,49 @@ def test_slices_in_one_workgroup(dev, m, n, k, split, nt, dtype):
     y = O.widen(y.view(np.float16) if dtype == "f16" else y, dtype)
     assert np.array_equal(y, O.widen(O.round_to(np.maximum(got, 0), dtype), dtype))
     # a larger result with the same rows and columns first takes the slices to the workspace: the same bits
-    big = 64 * 40
+    big = 32 * (dev.compute_units // -(-n // 32) + 1)
     a2 = np.zeros((big, k), a.dtype)
     a2[:m] = a
     ba2, bc2 = dev.buffer(a2.nbytes + 64, "device"), dev.buffer(4 * big * n, "device")
     ba2.upload(a2)
-    if -(-big // 32) * -(-n // 32) > 256:
-        mm(ba2, bb, bc2, big, n, k, bias=bbias)
-        assert np.array_equal(bc2.download(np.float32, (big, n))[:m], got)
+    assert mm.statistics(big, n, k)["workgroupThreads"] == 256
+    mm(ba2, bb, bc2, big, n, k, bias=bbias)
+    assert np.array_equal(bc2.download(np.float32, (big, n))[:m], got)
     for buf in (ba, bb, bbias, bc, by, ba2, bc2):
+        buf.destroy()
+
+
+@pytest.mark.parametrize("m,n,k,split,nt,lda,ldb,ldc,ldy", [
+    (33, 40, 200, 2, True, 208, 203, 43, 45), (70, 37, 256, 2, True, 264, 257, 40, 48),    # NT, B element by element
+    (33, 40, 264, 2, False, 272, 48, 44, 56), (65, 37, 328, 3, False, 336, 41, 37, 39),    # NN, pieces and elements
+    (64, 72, 520, 3, True, 528, 536, 80, 80), (32, 32, 128, 2, True, 136, 136, 33, 32)])   # NT, pieces
+@pytest.mark.parametrize("dtype", ["f16", "bf16"])
+def test_padded_pitches(dev, m, n, k, split, nt, lda, ldb, ldc, ldy, dtype):
+    """Integers, exact in any order; NaN between the rows of the operands, what lies between those of the results stays."""
+    from vkgrad_amd.kernels import Matmul
+    rng = np.random.default_rng(m + k)
+    a, b = rng.integers(-3, 4, (m, k)).astype(np.float32), rng.integers(-3, 4, (n, k) if nt else (k, n)).astype(np.float32)
+    bias, c0 = rng.integers(-9, 10, n).astype(np.float32), rng.integers(-9, 10, (m, ldc)).astype(np.float32)
+
+    def padded(x, pitch):
+        p = np.full((x.shape[0], pitch), np.nan, np.float32)
+        p[:, :x.shape[1]] = x
+        return O.round_to(p, dtype)
+    mm = Matmul(dev, trans_b=nt, dtype=dtype, tile=4, split_k=split)
+    assert mm.statistics(m, n, k, lda=lda, ldb=ldb, ldc=ldc)["workgroupThreads"] == 64 * split
+    pa, pb, y0 = padded(a, lda), padded(b, ldb), np.full((m, ldy), 7, np.uint16)
+    ba, bb, bbias, bc, by = bufs = [dev.buffer(x.nbytes, "device") for x in (pa, pb, bias, c0, y0)]
+    for buf, x in zip(bufs, (pa, pb, bias, c0, y0)):
+        buf.upload(x)
+    want = a @ (b.T if nt else b) + bias
+    mm(ba, bb, bc, m, n, k, bias=bbias, accumulate=True, lda=lda, ldb=ldb, ldc=ldc)
+    got = bc.download(np.float32, (m, ldc))
+    assert np.array_equal(got[:, :n], want + c0[:, :n]) and np.array_equal(got[:, n:], c0[:, n:])
+    mm(ba, bb, bc, m, n, k, bias=bbias, lda=lda, ldb=ldb, ldc=ldc, act="relu", y16=by, ldy=ldy)
+    got, y = bc.download(np.float32, (m, ldc)), by.download(np.uint16, (m, ldy))
+    assert np.array_equal(got[:, :n], want) and np.array_equal(got[:, n:], c0[:, n:]) and (y[:, n:] == 7).all()
+    assert np.array_equal(y[:, :n], O.round_to(np.maximum(want, 0), dtype).view(np.uint16))
+    for buf in bufs:
         buf.destroy()
 
 
