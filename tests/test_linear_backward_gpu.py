@@ -75,6 +75,59 @@ def test_exact_on_integers(dev, rows, fin, fout, tile, split_w, split_x, form, s
         buf.destroy()
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("tile,split_w,split_x,pad", [(4, 3, 2, 8), (11, 2, 2, 8), (21, 2, 2, 8), (4, 2, 1, 1), (4, 1, 3, 5)])
+@pytest.mark.parametrize("form", ["bias", "accumulate", "res", "act"])
+def test_padded_pitches_and_what_dx_adds(dev, tile, split_w, split_x, pad, form):
+    """Every matrix with a pitch of its own, NaN between the rows of the operands; dX onto its bias, onto itself, onto a residual, or
+    times the derivative with its column sums."""
+    if tile == 21 and form == "act":
+        form = "narrow"    # (those tiles have no derivative in one launch)
+    rows, fin, fout = (528, 264, 392) if pad == 8 else (301, 77, 139)
+    dtype = "f16" if (split_w + len(form)) % 2 else "bf16"
+    rng = np.random.default_rng(tile + pad)
+    data, host, bufs, pitch = {}, {}, {}, {}
+    shapes = dict(x=(rows, fin), w=(fin, fout), dy=(rows, fout), g32=(rows, fout), dw=(fin, fout), dx=(rows, fin), res=(rows, fin), z=(rows, fin),
+                  y=(rows, fin), bias=(1, fin), cs=(1, fin), db=(1, fout))
+    for i, (name, (r, c)) in enumerate(shapes.items()):
+        ld = pitch[name] = c if name in ("g32", "bias", "cs", "db") else c + pad * (1 + i % 3)
+        p = np.full((r, ld), np.nan if name in ("x", "w", "dy", "res", "z") else 5, np.float32)
+        data[name] = p[:, :c] = rng.integers(-3, 4, (r, c))
+        host[name] = O.round_to(p, dtype) if name in ("x", "w", "dy") else np.full((r, ld), 7, np.uint16) if name == "y" else p
+        bufs[name] = dev.buffer(host[name].nbytes + 16, "device")
+        bufs[name].upload(host[name])
+    B, P = bufs, pitch
+    gw = Matmul(None, trans_a=True, dtype=dtype)._args(B["x"], B["dy"], B["dw"], fin, fout, rows, 1, (0, 0, 0), None, True, P["x"], P["dy"], P["dw"])
+    extra = dict(bias=dict(bias=B["bias"]), accumulate=dict(accumulate=True), res=dict(res=B["res"], ldr=P["res"]),
+                 act=dict(act="relu_grad", z=B["z"], ldz=P["z"], y16=B["y"], ldy=P["y"], colsum=B["cs"]), narrow=dict(y16=B["y"], ldy=P["y"]))[form]
+    gx = Matmul(None, trans_b=True, dtype=dtype)._args(B["dy"], B["w"], B["dx"], rows, fin, fout, 1, (0, 0, 0), **{
+        **dict(bias=None, accumulate=False, lda=P["dy"], ldb=P["w"], ldc=P["dx"]), **extra})
+    b = L.BackwardArgs()
+    b.struct_size, b.tile, b.split_w, b.split_x, b.dw, b.dx = C.sizeof(b), tile, split_w, split_x, C.pointer(gw), C.pointer(gx)
+    b.g, b.db, b.rows, b.cols, b.g_f32 = B["g32"].ptr, B["db"].ptr, rows, fout, 1
+    _check(dev._lib.mg_gemm_backward(dev._ctx, C.byref(b)), "backward")
+    dev.sync()
+
+    def get(name):   # and what lies between the rows is as it was
+        got = bufs[name].download(host[name].dtype, host[name].shape)
+        c = shapes[name][1]
+        assert np.array_equal(got[:, c:], host[name][:, c:])
+        return got[:, :c]
+    assert np.array_equal(get("dw"), data["dw"] + data["x"].T @ data["dy"])
+    assert np.array_equal(get("db"), data["g32"].sum(0, keepdims=True))
+    want = data["dy"] @ data["w"].T
+    want += dict(bias=data["bias"], accumulate=data["dx"], res=data["res"]).get(form, 0)
+    if form == "act":
+        want *= data["z"] > 0
+        assert np.array_equal(get("cs"), data["cs"] + want.sum(0, keepdims=True))
+    if form in ("act", "narrow"):
+        y = get("y")
+        assert np.array_equal(O.widen(y.view(np.float16) if dtype == "f16" else y, dtype), O.widen(O.round_to(want.astype(np.float32), dtype), dtype))
+    assert np.array_equal(get("dx"), want)
+    for buf in bufs.values():
+        buf.destroy()
+
+
 class _Mem:
     host_visible, size = False, 1 << 40
 
