@@ -5,8 +5,21 @@ import numpy as np
 import pytest
 
 from oracle import ref_gemm as O
+from tests.test_flash_gpu import test_flash_attention as check
 
 pytestmark = pytest.mark.gpu
+
+
+# Every width class of a head (16, 32, 64, 96, 128; above 64 with one buffer a tensor), both directions, packed and not.
+@pytest.mark.parametrize("dtype,B,T,H,hd,packed", [
+    # 1405 blocks of 32 rows in 562 workgroups: whole rounds of 256, the second dealt out backwards, and a part of one
+    ("bf16", 1, 150, 281, 16, False), ("f16", 1, 150, 281, 32, False), ("bf16", 1, 150, 281, 64, False), ("f16", 1, 150, 281, 64, True),
+    ("bf16", 1, 150, 281, 80, True), ("f16", 1, 150, 281, 128, False),
+    # more than 1024 keys; with 15 heads and more, also too many blocks of 32 rows for the backward form of those
+    ("f16", 1, 1100, 1, 16, True), ("bf16", 1, 1100, 15, 32, True), ("bf16", 1, 1040, 17, 56, False), ("f16", 1, 1100, 15, 96, False),
+    ("bf16", 1, 1100, 1, 128, True)])
+def test_both_directions_of_every_width(B, T, H, hd, packed, dtype):
+    check(B, T, H, hd, packed, dtype)
 
 
 @pytest.mark.parametrize("gap", [60.0, 7.0, 0.0])
