@@ -1198,7 +1198,7 @@ int mg_tk_softmax_ce(mg_ctx *ctx, const float *logits, const uint32_t *labels, c
     if (ncls >= 16384) {   // a vocabulary
         kernel = f16 ? k_softmax_ce_wide<1024, MG_F16> : k_softmax_ce_wide<1024, MG_BF16>;
         threads = 1024;
-    } else if (ncls <= 1024) {   // all lanes of 256 threads would have a group of four: 16384 x 96 38 us so, 13.4 a wavefront each
+    } else if (ncls <= 1024) {   // all lanes of 256 threads would have a group of four: 16384 x 96 26 us so, 11.0 a wavefront each
         kernel = f16 ? k_softmax_ce_wide<64, MG_F16> : k_softmax_ce_wide<64, MG_BF16>;
         blocks = (unsigned)((nrows + 3) / 4);
     }
