@@ -38,6 +38,7 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 // 16 bytes with only 2-byte alignment promised: the hardware's unaligned access
 // mode serves these as a single dwordx4 load.
 typedef u32x4 __attribute__((aligned(2))) u32x4_u;
+typedef u32x4 __attribute__((aligned(4))) u32x4_d;
 
 struct GemmParams {
     const uint16_t *A;
@@ -152,7 +153,8 @@ __device__ __forceinline__ void tile_coords(const GemmParams &p, int &pid_m, int
 // extent (K for KC, the row count otherwise) a multiple of 8, so a chunk is
 // either entirely inside the matrix or entirely outside.
 // ---------------------------------------------------------------------------
-template <bool KC, int ROWS, int BK, int NTHREADS, bool GENERAL>
+// WHOLE (with GENERAL): blocks whose every row is there come by load_whole.
+template <bool KC, int ROWS, int BK, int NTHREADS, bool GENERAL, bool WHOLE = false>
 struct Stage {
     static constexpr int PITCH = KC ? (BK + 8) : (ROWS + 32);
     static constexpr int ELEMS = KC ? ROWS * PITCH : BK * PITCH;
@@ -163,9 +165,9 @@ struct Stage {
     static_assert(NCHUNK % NTHREADS == 0 && NTHREADS % CPR == 0, "tile/threads mismatch");
 
     u32x4 reg[PER];
-    // GENERAL: by how many elements each piece still has to move (load leaves it to store, one K-block later, so that
-    // nothing waits for a load at its issue), and whether any has to
-    int back[GENERAL ? PER : 1];
+    // GENERAL: by how many elements a thread's pieces still have to move (load leaves it to store, one K-block later, so that
+    // nothing waits for a load at its issue), how many of its LDS rows are there, and whether any of this matters
+    int back, there;
     bool edge = false;
 
     // Unconditional loads for a K-block that lies entirely inside the matrix in
@@ -179,6 +181,74 @@ struct Stage {
         for (int i = 0; i < PER; i++) {
             if constexpr (GENERAL) reg[i] = *(const u32x4_u *)(src + i * step);
             else reg[i] = *(const u32x4 *)(src + i * step);
+        }
+    }
+
+    // WHOLE, K-blocks whose every row is there: loads at dword addresses.  A 16-byte load at an address that is no multiple
+    // of 4 takes a CU's load path three to four times as long (from L2, KB a us and CU: rows of 128 bytes 150 where all are 16-byte
+    // aligned, 105 at multiples of 4, 38 at odd multiples of 2; of 256 bytes 170, 150, 39), so a piece that starts in the middle of a
+    // dword is fetched from the next dword (K-contiguous) or this one (else) and moved by 16 bits on its way to LDS.  The dword
+    // that it lacks is in the lane beside it; the first lane of a K-contiguous row has it from the row's last lane, one K-block
+    // earlier, the last lane of another row from `tail`, one load for all of the thread's rows together (a dword load a
+    // piece would cost as much as the piece).  Every dword read holds an element of the matrix.
+    uint32_t off[WHOLE ? PER : 1];                // bytes from the block's first dword
+    uint32_t toff, tail;
+    uint32_t carry[WHOLE && KC ? PER : 1];        // last dword of this lane's piece in the block before
+    uint32_t move;                                // what v_perm_b32 makes of two dwords for this thread's pieces
+    const char *at;                               // the block's first dword (uniform over the workgroup)
+
+    // Whether the offsets of a tile fit (pitches of millions of elements go the careful way).
+    static __device__ __forceinline__ bool offsets_fit(int64_t ld) { return ld < (1 << 21); }
+
+    // For a tile whose K-block kbeg is whole.  Rows (K-contiguous) or columns beyond the matrix repeat others of it: what
+    // they produce is masked; rows keep their parity, so that one `move` serves the thread.
+    __device__ __forceinline__ void whole_init(const uint16_t *base, int64_t ld, int row0, int nrows, int kbeg, int tid) {
+        static_assert(RSTEP % 2 == 0 && (!KC || CPR == 8), "a thread's rows are of one parity, and odd_piece");
+        const int r0 = tid / CPR, ch = tid % CPR;
+        const uint16_t *tile = KC ? base + (int64_t)row0 * ld + kbeg : base + (int64_t)kbeg * ld + row0;
+        const uint32_t first = (uint32_t)(uintptr_t)tile & 2;
+        at = reinterpret_cast<const char *>(tile) - first;
+        const int have = nrows - 1 - row0, last = have - ((have - r0) & 1);   // KC: last row of this parity, relative to the tile
+        auto row = [&](int i) { return !KC ? r0 + i * RSTEP : last < 0 ? 0 : min(r0 + i * RSTEP, last); };
+        auto bytes = [&](int i, int c) { return first + 2 * ((uint32_t)row(i) * (uint32_t)ld + (uint32_t)c); };
+        const bool odd = bytes(0, 0) & 2;
+        move = odd ? 0x05040302u : KC ? 0x07060504u : 0x03020100u;
+#pragma unroll
+        for (int i = 0; i < PER; i++) {
+            off[i] = KC ? (bytes(i, ch * 8) + 2) & ~3u : bytes(i, min(ch * 8, have)) & ~3u;
+            if constexpr (KC) carry[i] = *(const uint32_t *)(at + (bytes(i, 0) & ~3u));
+        }
+        // the dword behind the last piece of row i, for i as far from the last lane as this one (even pieces have no use for it)
+        const int i = min(CPR - 1 - ch, PER - 1);
+        toff = bytes(i, odd ? min(CPR * 8 - 8, have) + 8 : 0) & ~3u;
+    }
+    // TAIL: this operand has odd pieces
+    template <bool TAIL>
+    __device__ __forceinline__ void load_whole(int64_t step_bytes) {
+        edge = false;
+        asm("" : "+s"(at));   // a scalar base and lane offsets: the compiler would keep a 64-bit pointer a piece instead
+#pragma unroll
+        for (int i = 0; i < PER; i++) reg[i] = *(const u32x4_d *)(at + off[i]);
+        if constexpr (TAIL && !KC) tail = *(const uint32_t *)(at + toff);
+        at += step_bytes;
+    }
+    template <int I>
+    __device__ __forceinline__ u32x4 odd_piece(int tid) {
+        const u32x4 v = reg[I];
+        if constexpr (KC) {
+            // row_shr:1, and row_ror:9 from lane 7 to lane 0 and from 15 to 8
+            const uint32_t left = __builtin_amdgcn_update_dpp(0, (int)v[3], 0x111, 0xf, 0xf, false);
+            const uint32_t before = __builtin_amdgcn_update_dpp(0, (int)carry[I], 0x129, 0xf, 0xf, false);
+            carry[I] = v[3];
+            return u32x4{__builtin_amdgcn_perm(v[0], tid % CPR == 0 ? before : left, move), __builtin_amdgcn_perm(v[1], v[0], move),
+                         __builtin_amdgcn_perm(v[2], v[1], move), __builtin_amdgcn_perm(v[3], v[2], move)};
+        } else {
+            static_assert(I < CPR && I < 16, "the tails of a row's lanes");
+            // wave_shl:1 where a row of the tile takes 32 lanes, else row_shl:1; and row_shr:I
+            const uint32_t right = __builtin_amdgcn_update_dpp(0, (int)v[0], CPR > 16 ? 0x130 : 0x101, 0xf, 0xf, false);
+            const uint32_t t = I == 0 ? tail : (uint32_t)__builtin_amdgcn_update_dpp(0, (int)tail, 0x110 + I, 0xf, 0xf, false);
+            return u32x4{__builtin_amdgcn_perm(v[1], v[0], move), __builtin_amdgcn_perm(v[2], v[1], move),
+                         __builtin_amdgcn_perm(v[3], v[2], move), __builtin_amdgcn_perm(tid % CPR == CPR - 1 ? t : right, v[3], move)};
         }
     }
 
@@ -214,7 +284,7 @@ struct Stage {
         for (int i = 0; i < PER; i++) {
             const int c = tid + i * NTHREADS;
             u32x4 v = {0u, 0u, 0u, 0u};
-            if constexpr (GENERAL) back[i] = 0;
+            if constexpr (GENERAL) back = 0, there = BK;
             {
                 if constexpr (KC) {
                     const int r = c / CPR, kc = (c % CPR) * 8;
@@ -225,8 +295,8 @@ struct Stage {
                         if (k < kend) v = *(const u32x4 *)src;
                     } else if (kend >= 8) {
                         // the eight elements that end at kend, moved into place later: every lane issues one load, no branches
-                        back[i] = max(k + 8 - kend, 0);
-                        v = *(const u32x4_u *)(src - back[i]);
+                        back = max(k + 8 - kend, 0);
+                        v = *(const u32x4_u *)(src - back);
                     } else if (k < kend) {
                         v = chunk_elements(src, kend - k);
                     }
@@ -241,7 +311,7 @@ struct Stage {
                         if (nrows >= 8) {
                             const int b = max(row + 8 - nrows, 0);
                             v = *(const u32x4_u *)(base + (int64_t)min(k, kend - 1) * ld + row - b);
-                            back[i] = k < kend ? b : 8;
+                            back = b, there = kend - k0;
                         } else if (k < kend && row < nrows) {
                             v = chunk_elements(src, nrows - row);
                         }
@@ -252,21 +322,17 @@ struct Stage {
         }
     }
 
-    // WHOLE: the block is known to come from load_fast.
-    template <bool WHOLE = false>
-    __device__ __forceinline__ void store(uint16_t *lds, int tid) const {
-#pragma unroll
-        for (int i = 0; i < PER; i++) {
-            const int c = tid + i * NTHREADS;
-            {
-                const int r = c / CPR, off = (c % CPR) * 8;
-                if constexpr (GENERAL && !WHOLE) {
-                    *(u32x4 *)(lds + r * PITCH + off) = edge ? chunk_shift(reg[i], back[i]) : reg[i];
-                } else {
-                    *(u32x4 *)(lds + r * PITCH + off) = reg[i];
-                }
-            }
-        }
+    // FROM 0: whatever load the block came from; 1: load_fast, or load_whole with even pieces; 2: load_whole.
+    template <int FROM = 0, int I = 0>
+    __device__ __forceinline__ void store(uint16_t *lds, int tid) {
+        const int c = tid + I * NTHREADS;
+        u32x4 *to = (u32x4 *)(lds + c / CPR * PITCH + (c % CPR) * 8);
+        if constexpr (!GENERAL || FROM == 1) *to = reg[I];
+        else if constexpr (FROM == 2) *to = odd_piece<I>(tid);
+        else if (edge) *to = chunk_shift(reg[I], KC || c / CPR < there ? back : 8);
+        else if constexpr (WHOLE) *to = odd_piece<I>(tid);
+        else *to = reg[I];
+        if constexpr (I + 1 < PER) store<FROM, I + 1>(lds, tid);
     }
 
     // One 32-row x 16-k MFMA operand fragment: lane l gets row (l % 32),
@@ -727,8 +793,10 @@ __device__ __forceinline__ void gemm_body(const GemmParams &p, int tile, int sli
     constexpr int TM = WTM / 32, TN = WTN / 32;
     constexpr int KK = BK / 16;
     static_assert(WTM % 32 == 0 && WTN % 32 == 0 && BK % 32 == 0, "tile shape");
-    using SA = Stage<A_KC, BM, BK, NTHREADS, GENERAL>;
-    using SB = Stage<B_KC, BN, BK, NTHREADS, GENERAL>;
+    // (beside the accumulators of the 256 x 256 tile there is no room for its offsets)
+    constexpr bool WHOLE = GENERAL && BM * BN < 256 * 256;
+    using SA = Stage<A_KC, BM, BK, NTHREADS, GENERAL, WHOLE>;
+    using SB = Stage<B_KC, BN, BK, NTHREADS, GENERAL, WHOLE>;
     constexpr int STAGE_ELEMS = SA::ELEMS + SB::ELEMS;
     // LDS read instructions per fragment: one b128, or two transposing b64
     constexpr int NDSR = TM * (A_KC ? 1 : 2) + TN * (B_KC ? 1 : 2);
@@ -755,10 +823,20 @@ __device__ __forceinline__ void gemm_body(const GemmParams &p, int tile, int sli
     // an empty slice has nothing to add to C, except the bias when it is the slice that carries it
     if (kend == kbeg && p.split_k > 1 && p.ws == nullptr && !(p.bias != nullptr && slice == 0)) return;
     const int nkb = (kend - kbeg + BK - 1) / BK;
-    // K-blocks that the unconditional loader may fetch: the whole block inside
-    // K, and the tile inside M and N.
+    // K-blocks that the unconditional loader may fetch: the whole block inside K, and the tile inside M and N.  At any
+    // alignment it takes tiles at the edges too: rows of a K-contiguous operand repeat, and a piece of columns beyond the
+    // matrix runs on into the next row - into every row but the last.
     const bool interior = (m0 + BM <= p.M) && (n0 + BN <= p.N);
-    const int nkb_fast = interior ? (kend - kbeg) / BK : 0;
+    int nkb_fast = WHOLE || interior ? (kend - kbeg) / BK : 0;
+    bool odd_a = false, odd_b = false;   // some piece starts in the middle of a dword
+    if constexpr (WHOLE) {
+        auto edge_blocks = [&](int64_t ld) { return ld >= 16 ? (p.K - 1 - kbeg) / BK : 0; };
+        if (!A_KC && m0 + BM > p.M) nkb_fast = min(nkb_fast, edge_blocks(p.lda));
+        if (!B_KC && n0 + BN > p.N) nkb_fast = min(nkb_fast, edge_blocks(p.ldb));
+        if (!SA::offsets_fit(p.lda) || !SB::offsets_fit(p.ldb)) nkb_fast = 0;
+        odd_a = (p.lda & 1) || ((uintptr_t)A & 2);
+        odd_b = (p.ldb & 1) || ((uintptr_t)B & 2);
+    }
 
     f32x16 acc[TM][TN];
 #pragma unroll
@@ -781,10 +859,26 @@ __device__ __forceinline__ void gemm_body(const GemmParams &p, int tile, int sli
         const int64_t k0 = kbeg + (int64_t)kb * BK;
         return B_KC ? B + (int64_t)n0 * p.ldb + k0 : B + k0 * p.ldb + n0;
     };
-    auto load_block = [&](int kb) {   // uniform branch: fast when the block is interior
-        if (kb < nkb_fast) {
+    const int64_t a_step = (A_KC ? BK : BK * p.lda) * 2, b_step = (B_KC ? BK : BK * p.ldb) * 2;
+    if (WHOLE && nkb_fast > 0) {
+        if constexpr (WHOLE) {
+            sa.whole_init(A, p.lda, m0, p.M, kbeg, tid);
+            sb.whole_init(B, p.ldb, n0, p.N, kbeg, tid);
+        }
+    }
+    // (whole blocks come in order)
+    auto load_fast = [&](auto mode, int kb) {
+        if constexpr (WHOLE) {
+            sa.template load_whole<(decltype(mode)::value & 2) != 0>(a_step);
+            sb.template load_whole<(decltype(mode)::value & 4) != 0>(b_step);
+        } else {
             sa.load_fast(a_tile(kb), p.lda, tid);
             sb.load_fast(b_tile(kb), p.ldb, tid);
+        }
+    };
+    auto load_block = [&](int kb) {   // uniform branch: fast when the block is interior
+        if (kb < nkb_fast) {
+            load_fast(IntC<7>{}, kb);
         } else {
             sa.load(A, p.lda, m0, p.M, kbeg + kb * BK, kend, tid);
             sb.load(B, p.ldb, n0, p.N, kbeg + kb * BK, kend, tid);
@@ -816,8 +910,8 @@ __device__ __forceinline__ void gemm_body(const GemmParams &p, int tile, int sli
     if (nkb > 0) read_frags(smem, 0, 0);
 
     // One K-block.  MODE 1: blocks kb+1 and kb+2 exist and kb+2 is interior, so
-    // the loop body is straight-line code; MODE 0: generic tail with uniform
-    // branches.  The global loads issued here are consumed one whole K-block
+    // the loop body is straight-line code (MODE 3, 5, 7: with odd pieces of A, of B, of both); MODE 0: generic tail with
+    // uniform branches.  The global loads issued here are consumed one whole K-block
     // later, by the LDS writes of the next iteration.
     auto kblock = [&](auto mode, int kb) {
         constexpr int MODE = decltype(mode)::value;
@@ -828,24 +922,23 @@ __device__ __forceinline__ void gemm_body(const GemmParams &p, int tile, int sli
             const int cur = kk & 1, nxt = cur ^ 1;
             if (kk < KK - 1) {
                 read_frags(As, kk + 1, nxt);
-            } else if (MODE == 1 || kb + 1 < nkb) {
+            } else if (MODE || kb + 1 < nkb) {
                 read_frags(An, 0, nxt);   // next stage is complete: the barrier below has passed
             }
             if (kk == KK - 2) {
-                if (MODE == 1 || kb + 1 < nkb) {
-                    sa.template store<MODE == 1>(An, tid);
-                    sb.template store<MODE == 1>(An + SA::ELEMS, tid);
+                if (MODE || kb + 1 < nkb) {
+                    sa.template store<MODE == 0 ? 0 : MODE & 2 ? 2 : 1>(An, tid);
+                    sb.template store<MODE == 0 ? 0 : MODE & 4 ? 2 : 1>(An + SA::ELEMS, tid);
                 }
-                if constexpr (MODE == 1) {
-                    sa.load_fast(a_tile(kb + 2), p.lda, tid);
-                    sb.load_fast(b_tile(kb + 2), p.ldb, tid);
+                if constexpr (MODE) {
+                    load_fast(IntC<MODE>{}, kb + 2);
                 } else {
                     if (kb + 2 < nkb) load_block(kb + 2);
                 }
             }
             mfma_group(cur);
-            if constexpr (MODE == 1) {
-                if (kk == KK - 2) interleave_group<TM * TN, NDSR, NLOAD, NLOAD>();
+            if constexpr (MODE) {
+                if (kk == KK - 2) interleave_group<TM * TN, NDSR, NLOAD, NLOAD + (MODE & 2 && !A_KC) + (MODE & 4 && !B_KC)>();
                 else interleave_group<TM * TN, NDSR, 0, 0>();
             }
             if (kk == KK - 2) __syncthreads();
@@ -854,7 +947,17 @@ __device__ __forceinline__ void gemm_body(const GemmParams &p, int tile, int sli
 
     int kb = 0;
     const int n_steady = nkb_fast - 2;   // iterations whose kb+2 prefetch is interior
-    for (; kb < n_steady; kb++) kblock(IntC<1>{}, kb);
+    auto steady = [&](auto mode) {
+        for (; kb < n_steady; kb++) kblock(mode, kb);
+    };
+    // (odd pieces of a K-contiguous operand cost a few moves, others a load too: loops of their own for one of two of those)
+    if (!WHOLE || (!odd_a && !odd_b)) {
+        steady(IntC<1>{});
+    } else if constexpr (WHOLE) {
+        if (LAYOUT == L_TN && !odd_b) steady(IntC<LAYOUT == L_TN ? 3 : 7>{});
+        else if (LAYOUT == L_TN && !odd_a) steady(IntC<LAYOUT == L_TN ? 5 : 7>{});
+        else steady(IntC<7>{});
+    }
     for (; kb < nkb; kb++) kblock(IntC<0>{}, kb);
 
     // Epilogue.  Accumulator register r of lane l holds
@@ -890,7 +993,7 @@ __device__ __forceinline__ void gemm_body(const GemmParams &p, int tile, int sli
 }
 
 template <int LAYOUT, int DT, int BM, int BN, int BK, int WGM, int WGN, bool GENERAL, bool ACT = false>
-__global__ void __launch_bounds__(WGM *WGN * 64, (ACT && BM * BN == 128 * 128 ? 2 : 1))   // (two workgroups a CU: 256 registers, not 260)
+__global__ void __launch_bounds__(WGM *WGN * 64, (GENERAL && BM * BN <= 128 * 128 ? 2 : 1))   // (two workgroups a CU: 256 registers, not 260)
 gemm_kernel(const GemmParams p) {
     extern __shared__ __attribute__((aligned(16))) uint16_t smem[];
     gemm_body<LAYOUT, DT, BM, BN, BK, WGM, WGN, GENERAL, ACT>(p, blockIdx.x, blockIdx.y, smem);
