@@ -143,11 +143,6 @@ __global__ void k_copy(const uint32_t *src, uint32_t *dst, int64_t nwords, int v
 // training as it did: an add of a lane's value every few clocks, 0.4 us for 100 classes.  Beyond, where it would be the
 // longest part of the kernel, the lanes' partial sums meet in a tree.
 constexpr int CE_IN_ORDER = 128;
-__device__ __forceinline__ float ce_wave_sum(float v) {
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) v += __shfl_xor(v, m, 64);
-    return v;
-}
 __global__ void __launch_bounds__(256) k_softmax_ce(const float *logits, const uint32_t *labels, uint16_t *dl16, float *dl32,
                                                     float *loss, int64_t nrows, int64_t stride, int64_t ncls, int dtype) {
     const int lane = threadIdx.x & 63;
@@ -157,8 +152,7 @@ __global__ void __launch_bounds__(256) k_softmax_ce(const float *logits, const u
     const float x0 = lane < ncls ? row[lane] : -1e30f;   // a row of up to 64 classes stays in registers
     float mx = x0;
     for (int64_t c = lane + 64; c < ncls; c += 64) mx = fmaxf(mx, row[c]);
-#pragma unroll
-    for (int m = 32; m >= 1; m >>= 1) mx = fmaxf(mx, __shfl_xor(mx, m, 64));
+    mx = wave_max(mx);
     float s = lane < ncls ? expf(x0 - mx) : 0.f;
     if (ncls <= CE_IN_ORDER) {
         // in the order of the classes, lane by lane: the sum of a serial loop to the last bit
@@ -171,7 +165,7 @@ __global__ void __launch_bounds__(256) k_softmax_ce(const float *logits, const u
         s = t;
     } else {
         for (int64_t c = lane + 64; c < ncls; c += 64) s += expf(row[c] - mx);
-        s = ce_wave_sum(s);
+        s = wave_sum(s);
     }
     const float logZ = mx + logf(s);
     const int64_t y = labels[i];

@@ -36,6 +36,33 @@ __device__ __forceinline__ uint32_t pack16(float a, float b) {
     else return __builtin_bit_cast(uint32_t, b2{(__bf16)a, (__bf16)b});
 }
 
+// What all 64 lanes of a wavefront hold, combined by a commutative f (in all of them): with the value 32, 16, 8, 4, 2 and 1
+// lanes away in turn, the order - and so the bits - of a butterfly of __shfl_xor, but in VALU moves (v_permlane32_swap, v_permlane16_swap, DPP
+// rotations within 16 lanes) instead of six LDS round trips of 100 clocks and more, one behind the other.
+template <int CTRL>
+__device__ __forceinline__ float wave_dpp(float v) {
+    const int i = __builtin_bit_cast(int, v);
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(i, i, CTRL, 0xf, 0xf, false));
+}
+template <class F>
+__device__ __forceinline__ float wave_all(float v, F f) {
+    const auto pair = [&](auto r) { return f(__builtin_bit_cast(float, (uint32_t)r[0]), __builtin_bit_cast(float, (uint32_t)r[1])); };
+    uint32_t u = __builtin_bit_cast(uint32_t, v);
+    v = pair(__builtin_amdgcn_permlane32_swap(u, u, false, false));
+    u = __builtin_bit_cast(uint32_t, v);
+    v = pair(__builtin_amdgcn_permlane16_swap(u, u, false, false));
+    v = f(v, wave_dpp<0x128>(v));   // row_ror:8
+    v = f(v, wave_dpp<0x124>(v));   // row_ror:4, of values that repeat every 8 lanes
+    v = f(v, wave_dpp<0x4e>(v));    // quad_perm 2 3 0 1
+    return f(v, wave_dpp<0xb1>(v)); // quad_perm 1 0 3 2
+}
+__device__ __forceinline__ float wave_sum(float v) {
+    return wave_all(v, [](float a, float b) { return a + b; });
+}
+__device__ __forceinline__ float wave_max(float v) {
+    return wave_all(v, [](float a, float b) { return fmaxf(a, b); });
+}
+
 // Column sums: rows of a chunk - several chunks add with atomics -, and how many rows of an f32 matrix one chunk of
 // twice the threads takes at the most.  The sums that share a launch with products (gemm_backward_kernel.h) have the same chunks, and so
 // the same bits.
