@@ -234,6 +234,39 @@ def test_whose_plans_bind(monkeypatch):
         assert recorded(mm, Matmul(Dev(), trans_b=True, split_k=2)) == L.MG_BACKWARD_AUTO
 
 
+def test_how_slices_of_a_shipped_plan_meet(monkeypatch):
+    """Slices that add with atomics keep a pass in turn where the caller asked for them, not where a shipped plan has them."""
+    from vkgrad_amd import kernels as K
+    from vkgrad_amd.autograd import Ctx
+
+    class Dev:
+        _lib, _ctx, name, compute_units = L.load(), None, "fake", 256
+
+    key = K.tune_key("fake", 1024, 256, 16384, True, False)
+    table = {key: {"tile_id": 14, "split_k": 15, "group_m": 4, "atomic_split": True}}
+    monkeypatch.setattr(K, "_shipped_table", lambda: table)
+    monkeypatch.setattr(K, "_load_cache", lambda path=None: {})
+    ctx = Ctx.__new__(Ctx)
+    ctx.dev, ctx.tune, ctx.dtype, ctx._mm = Dev(), False, "f16", {}
+    shipped = ctx.matmul(1024, 256, 16384, trans_a=True)
+    assert shipped.atomic_split and shipped.from_table
+    bufs = {n: _Mem((i + 1) << 33) for i, n in enumerate(("x", "w", "dy", "dw", "z", "y"))}
+
+    def pick(mw, mx=None):
+        g = Graph(Dev(), "g")
+        linear_backward(Dev(), (mw, (bufs["x"], bufs["dy"], bufs["dw"], 1024, 256, 16384), {}),
+                        (mx or Matmul(Dev(), trans_b=True), (bufs["dy"], bufs["w"], None, 16384, 1024, 256),
+                         dict(act="gelu_grad", z=bufs["z"], y16=bufs["y"])), graph=g)
+        ba, out = g._thunks[0].__defaults__[0], [C.c_int() for _ in range(3)]
+        assert Dev._lib.mg_backward_pick(C.byref(ba), 256, *(C.byref(o) for o in out)) == L.MG_OK
+        return ba.dw.contents.flags & L.MG_FLAG_SPLITK_ATOMIC, out[0].value
+
+    flag, tile = pick(shipped)
+    assert flag == 0 and tile in (4, 11)
+    named = Matmul(Dev(), trans_a=True, tile=14, split_k=15, atomic_split=True)
+    assert pick(named) == (L.MG_FLAG_SPLITK_ATOMIC, L.MG_BACKWARD_APART)
+
+
 def test_keywords_of_a_product_arrive():
     """Every keyword of Matmul's call reaches the product, with its buffer; others are refused."""
     class Dev:
