@@ -200,7 +200,7 @@ constexpr int dma_waves_per_simd() {
 }
 
 // One workgroup's share of a product: tile number `tile` (of grid_m * grid_n, before renumbering) of K slice `slice`.
-template <int LAYOUT, int DT, int BM, int BN, int BK, int WGM, int WGN, int NSTAGE, bool ACT>
+template <int LAYOUT, int DT, int BM, int BN, int BK, int WGM, int WGN, int NSTAGE, bool ACT, int WAVES = 0>
 __device__ __forceinline__ void gemm_dma_body(const GemmParams &p, int tile, int slice, char *dsm) {
     constexpr bool A_KC = (LAYOUT != L_TN);
     constexpr bool B_KC = (LAYOUT == L_NT);
@@ -410,19 +410,25 @@ __device__ __forceinline__ void gemm_dma_body(const GemmParams &p, int tile, int
     if constexpr (ACT) {
         static_assert(WGM * WGN * 32 * (WTN + 8) * 4 <= NSTAGE * STAGE_BYTES, "row pieces fit the ring");
         if (p.rows16 && mode != 2 && (TM * TN <= 4 || p.act < 3)) {
-            store_tile_rows<DT, TM, TN, WTM, WTN, WGM * WGN>(p, p.C ? C : nullptr, acc, m0, n0, wave, wave_m, wave_n, lane, add_bias,
-                                                             mode, reinterpret_cast<char *>(dsm));
+            constexpr bool TIGHT = WAVES > 2;
+            store_tile_rows<DT, TM, TN, WTM, WTN, WGM * WGN, TIGHT>(p, p.C ? C : nullptr, acc, m0, n0, wave, wave_m, wave_n, lane,
+                                                                    add_bias, mode, reinterpret_cast<char *>(dsm));
             return;
         }
     }
     store_tile<DT, TM, TN, WTM, WTN, ACT>(p, C, acc, m0, n0, wave_m, wave_n, lane, add_bias, mode, interior);
 }
 
-template <int LAYOUT, int DT, int BM, int BN, int BK, int WGM, int WGN, int NSTAGE, bool ACT = false>
-__global__ void __launch_bounds__(WGM *WGN * 64, (dma_waves_per_simd<BM, BN, BK, WGM, WGN, NSTAGE>()))
+// WAVES: wavefronts a SIMD is to hold, where it is not what the tile has by itself.  The 128 x 128 tile with K-blocks of 32 takes 48 KB of
+// LDS and, left alone, 220 registers: two workgroups a CU.  Held under 170 (127, 166 with the fused outputs, no spills) a third one
+// multiplies while others fill their ring or store, where the product has more than two for a CU.  bf16: 8192 x 3072 x 768 with GELU
+// 74 -> 64 us, 8192 x 2304 x 768 to 16 bits 44 -> 40, 16384 x 768 x 256 16.7 -> 14.4, onto a residual 32.0 -> 28.6; with
+// two or fewer the times are the same (8192 x 768 x 3072 54.7), and the fused outputs keep their longer steps.
+template <int LAYOUT, int DT, int BM, int BN, int BK, int WGM, int WGN, int NSTAGE, bool ACT = false, int WAVES = 0>
+__global__ void __launch_bounds__(WGM *WGN * 64, (WAVES ? WAVES : dma_waves_per_simd<BM, BN, BK, WGM, WGN, NSTAGE>()))
 gemm_dma_kernel(const GemmParams p) {
     extern __shared__ __attribute__((aligned(1024))) char dsm[];
-    gemm_dma_body<LAYOUT, DT, BM, BN, BK, WGM, WGN, NSTAGE, ACT>(p, blockIdx.x, blockIdx.y, dsm);
+    gemm_dma_body<LAYOUT, DT, BM, BN, BK, WGM, WGN, NSTAGE, ACT, WAVES>(p, blockIdx.x, blockIdx.y, dsm);
 }
 
 // ---------------------------------------------------------------------------
@@ -774,10 +780,10 @@ gemm_dmap_kernel(const GemmParams p) {
     }
 }
 
-template <int LAYOUT, int DT, int BM, int BN, int BK, int WGM, int WGN, int NSTAGE, bool ACT = false>
+template <int LAYOUT, int DT, int BM, int BN, int BK, int WGM, int WGN, int NSTAGE, bool ACT = false, int WAVES = 0>
 hipError_t launch_gemm_dma(const GemmParams &p, dim3 grid, hipStream_t stream, KernelQuery *query = nullptr) {
     using TT = DmaTraits<LAYOUT, BM, BN, BK, WGM, WGN, NSTAGE>;
-    auto kern = gemm_dma_kernel<LAYOUT, DT, BM, BN, BK, WGM, WGN, NSTAGE, ACT>;
+    auto kern = gemm_dma_kernel<LAYOUT, DT, BM, BN, BK, WGM, WGN, NSTAGE, ACT, WAVES>;
     static std::atomic<uint64_t> lds_allowed{0};
     hipError_t e = allow_dynamic_lds((const void *)kern, TT::LDS_BYTES, lds_allowed);
     if (e != hipSuccess) return e;

@@ -5,6 +5,7 @@
 // Entry [tile][2] is the variant whose epilogue also writes the activated 16-bit output
 // (forward layouts NN and NT, tiles 3, 4, 10, 11, 14 and 21; null elsewhere); tiles 3 and 4 have
 // it for any alignment, and in [3] for aligned operands with direct loads.
+// Entries [tile][3] and [4] of a direct-to-LDS tile are those of [2] and [0] for three workgroups a CU (tile 14).
 #include "gemm_dma_kernel.h"
 #include "gemm_pp_kernel.h"
 #include "gemm_kernel.h"
@@ -32,6 +33,11 @@ constexpr launch_fn act_variant_d() {
     if constexpr ((ID == 10 || ID == 11 || ID == 14) && L_NN != L_TN) return launch_gemm_dma<L_NN, D_BF16, BM, BN, BK, WGM, WGN, NS, true>;
     else return nullptr;
 }
+template <int ID, int BM, int BN, int BK, int WGM, int WGN, int NS, bool ACT>
+constexpr launch_fn three_variant_d() {
+    if constexpr (ID == 14 && !(ACT && L_NN == L_TN)) return launch_gemm_dma<L_NN, D_BF16, BM, BN, BK, WGM, WGN, NS, ACT, 3>;
+    else return nullptr;
+}
 template <int BM, int BN, int BK, int WGM, int WGN>
 constexpr launch_fn act_variant_q() {
     if constexpr (L_NN != L_TN) return launch_gemm_pp<L_NN, D_BF16, BM, BN, BK, WGM, WGN, true>;
@@ -50,7 +56,8 @@ constexpr launch_fn bias_variant_p() {
     {aligned_variant_v<id, bm, bn, bk, wgm, wgn>(), launch_gemm<L_NN, D_BF16, bm, bn, bk, wgm, wgn, true>, \
      act_variant_v<id, bm, bn, bk, wgm, wgn>(), act_aligned_variant_v<id, bm, bn, bk, wgm, wgn>()},
 #define D(id, bm, bn, bk, wgm, wgn, ns, fb) \
-    {launch_gemm_dma<L_NN, D_BF16, bm, bn, bk, wgm, wgn, ns>, nullptr, act_variant_d<id, bm, bn, bk, wgm, wgn, ns>()},
+    {launch_gemm_dma<L_NN, D_BF16, bm, bn, bk, wgm, wgn, ns>, nullptr, act_variant_d<id, bm, bn, bk, wgm, wgn, ns>(), \
+     three_variant_d<id, bm, bn, bk, wgm, wgn, ns, true>(), three_variant_d<id, bm, bn, bk, wgm, wgn, ns, false>()},
 #define P(id, bm, bn, bk, wgm, wgn, ns, fb)                          \
     {launch_gemm_dmap<L_NN, D_BF16, bm, bn, bk, wgm, wgn, ns, false, false>, \
      bias_variant_p<bm, bn, bk, wgm, wgn, ns, false>(), nullptr},
@@ -61,7 +68,7 @@ constexpr launch_fn bias_variant_p() {
 #define S(id, bm, bn, bk, wgm, wgn, ns, fb)                                \
     {launch_gemm_dmap<L_NN, D_BF16, bm, bn, bk, wgm, wgn, ns, false, true>, \
      bias_variant_p<bm, bn, bk, wgm, wgn, ns, true>(), nullptr},
-launch_fn launch_table_nn_bf16[MG_NUM_TILES][4] = {MG_TILE_LIST(V, D, P, S, G, Q, W)};
+launch_fn launch_table_nn_bf16[MG_NUM_TILES][5] = {MG_TILE_LIST(V, D, P, S, G, Q, W)};
 #undef V
 #undef D
 #undef P

@@ -660,14 +660,14 @@ __device__ __forceinline__ void store_tile(const GemmParams &p, float *C, f32x16
 // of Z, R or C.  The pitch of WTN + 8 floats puts the two half-waves' rows on different banks.
 // ACTV: MG_ACT_*, known at compile time - a test of it per element would put every exponential in a basic block
 // of its own, one dependent chain after the other.
-template <int DT, int TM, int TN, int WTM, int WTN, int NW, int ACTV>
+template <int DT, int TM, int TN, int WTM, int WTN, int NW, bool TIGHT, int ACTV>
 __device__ __forceinline__ void store_tile_rows(const GemmParams &p, float *C, f32x16 (&acc)[TM][TN], int m0, int n0,
                                                 int wave, int wave_m, int wave_n, int lane, bool add_bias, int mode, char *lds) {
     constexpr int PITCH = WTN + 8;            // floats
     constexpr int LPR = WTN / 8;              // lanes per row
     constexpr int RPI = 64 / LPR;             // rows per step
-    // steps taken together: a whole strip of 32 rows, half of one where the accumulators leave fewer registers
-    constexpr int NK = 32 / RPI / (TM * TN > 4 ? 2 : 1);
+    // steps taken together: a whole strip of 32 rows, half of one where the accumulators, or three workgroups a CU, leave fewer registers
+    constexpr int NK = 32 / RPI / (TM * TN > 4 || TIGHT ? 2 : 1);
     constexpr int HALVES = 32 / RPI / NK;
     constexpr bool GRAD = ACTV == 3 || ACTV == 4;
     typedef float f4 __attribute__((ext_vector_type(4)));
@@ -767,11 +767,11 @@ __device__ __forceinline__ void store_tile_rows(const GemmParams &p, float *C, f
         }
     }
 }
-template <int DT, int TM, int TN, int WTM, int WTN, int NW>
+template <int DT, int TM, int TN, int WTM, int WTN, int NW, bool TIGHT = false>
 __device__ __forceinline__ void store_tile_rows(const GemmParams &p, float *C, f32x16 (&acc)[TM][TN], int m0, int n0,
                                                 int wave, int wave_m, int wave_n, int lane, bool add_bias, int mode, char *lds) {
     auto run = [&](auto act_c) {
-        store_tile_rows<DT, TM, TN, WTM, WTN, NW, decltype(act_c)::value>(p, C, acc, m0, n0, wave, wave_m, wave_n, lane, add_bias,
+        store_tile_rows<DT, TM, TN, WTM, WTN, NW, TIGHT, decltype(act_c)::value>(p, C, acc, m0, n0, wave, wave_m, wave_n, lane, add_bias,
                                                                           mode, lds);
     };
     if constexpr (TM * TN <= 4) {   // (beside the accumulators of a 128 x 64 wavefront tile the derivatives spill)
