@@ -39,6 +39,11 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 // mode serves these as a single dwordx4 load.
 typedef u32x4 __attribute__((aligned(2))) u32x4_u;
 typedef u32x4 __attribute__((aligned(4))) u32x4_d;
+// Global memory, where a pointer passes through something that hides where it points to (an asm statement): a load
+// through a generic pointer is a flat one, which LDS waits count as well.
+typedef const __attribute__((address_space(1))) char glb_char_t;
+typedef const __attribute__((address_space(1))) uint32_t glb_u32_t;
+typedef const __attribute__((address_space(1))) u32x4_d glb_u32x4_d;
 
 struct GemmParams {
     const uint16_t *A;
@@ -195,7 +200,7 @@ struct Stage {
     uint32_t toff, tail;
     uint32_t carry[WHOLE && KC ? PER : 1];        // last dword of this lane's piece in the block before
     uint32_t move;                                // what v_perm_b32 makes of two dwords for this thread's pieces
-    const char *at;                               // the block's first dword (uniform over the workgroup)
+    glb_char_t *at;                               // the block's first dword (uniform over the workgroup)
 
     // Whether the offsets of a tile fit (pitches of millions of elements go the careful way).
     static __device__ __forceinline__ bool offsets_fit(int64_t ld) { return ld < (1 << 21); }
@@ -207,7 +212,7 @@ struct Stage {
         const int r0 = tid / CPR, ch = tid % CPR;
         const uint16_t *tile = KC ? base + (int64_t)row0 * ld + kbeg : base + (int64_t)kbeg * ld + row0;
         const uint32_t first = (uint32_t)(uintptr_t)tile & 2;
-        at = reinterpret_cast<const char *>(tile) - first;
+        at = (glb_char_t *)(tile) - first;
         const int have = nrows - 1 - row0, last = have - ((have - r0) & 1);   // KC: last row of this parity, relative to the tile
         auto row = [&](int i) { return !KC ? r0 + i * RSTEP : last < 0 ? 0 : min(r0 + i * RSTEP, last); };
         auto bytes = [&](int i, int c) { return first + 2 * ((uint32_t)row(i) * (uint32_t)ld + (uint32_t)c); };
@@ -216,7 +221,7 @@ struct Stage {
 #pragma unroll
         for (int i = 0; i < PER; i++) {
             off[i] = KC ? (bytes(i, ch * 8) + 2) & ~3u : bytes(i, min(ch * 8, have)) & ~3u;
-            if constexpr (KC) carry[i] = *(const uint32_t *)(at + (bytes(i, 0) & ~3u));
+            if constexpr (KC) carry[i] = *(glb_u32_t *)(at + (bytes(i, 0) & ~3u));
         }
         // the dword behind the last piece of row i, for i as far from the last lane as this one (even pieces have no use for it)
         const int i = min(CPR - 1 - ch, PER - 1);
@@ -228,8 +233,8 @@ struct Stage {
         edge = false;
         asm("" : "+s"(at));   // a scalar base and lane offsets: the compiler would keep a 64-bit pointer a piece instead
 #pragma unroll
-        for (int i = 0; i < PER; i++) reg[i] = *(const u32x4_d *)(at + off[i]);
-        if constexpr (TAIL && !KC) tail = *(const uint32_t *)(at + toff);
+        for (int i = 0; i < PER; i++) reg[i] = *(glb_u32x4_d *)(at + off[i]);
+        if constexpr (TAIL && !KC) tail = *(glb_u32_t *)(at + toff);
         at += step_bytes;
     }
     template <int I>
