@@ -353,8 +353,9 @@ typedef struct {
 int mg_kernel_stats_for(mg_ctx *ctx, const mg_gemm_args *args, int *tile, mg_kernel_stats *out);
 /* The same for one instantiation named directly: tile id, layout (MG_NN..), dtype, and
  * variant 0 (aligned operands / plain epilogue), 1 (any alignment for register-staged tiles,
- * bias epilogue for persistent ones) or 2 (fused activation output).  For the skinny-M tile the
- * variant is 4 * log2(rows of A held) + K class (0: K <= 512, 1: 768, 2: 1024, 3: 2048).
+ * bias epilogue for persistent ones), 2 (fused activation output), 3 (the same with direct loads
+ * for register-staged tiles, for three workgroups a CU for direct-to-LDS ones) or 4 (aligned
+ * operands, for three workgroups a CU).  For the skinny-M tile the variant is 4 * log2(rows of A held) + K class (0: K <= 512, 1: 768, 2: 1024, 3: 2048).
  * MG_ERR_ARG when the table holds no such instantiation. */
 int mg_tile_kernel_stats(mg_ctx *ctx, int tile, int layout, int dtype, int variant, mg_kernel_stats *out);
 /* Matmul.fits for one tile: 1 if tile `id` can run `args`, else 0. */

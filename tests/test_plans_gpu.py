@@ -365,7 +365,7 @@ def test_no_instantiation_spills_and_occupancy_is_as_designed(dev):
         skinny = t["name"].startswith(("mv_", "ms_"))
         for layout in (K.L.MG_NN, K.L.MG_NT, K.L.MG_TN):
             for dtype in ("f16", "bf16"):
-                for variant in (range(16) if skinny else range(3)):
+                for variant in (range(16) if skinny else range(5)):
                     st = K.tile_statistics(dev, t["id"], layout, dtype, variant)
                     if st is None:
                         continue
@@ -378,7 +378,9 @@ def test_no_instantiation_spills_and_occupancy_is_as_designed(dev):
                         continue
                     assert st["workgroupThreads"] == t["threads"], what
                     assert st["ldsUsageSizeInBytes"] <= 160 * 1024, what
-                    if t["name"] in _WGS_PER_CU:
+                    if t["name"] == "mmd_128x128x32_w2x2_s3" and variant >= 3:   # its form for three workgroups a CU
+                        assert st["workgroupsPerCU"] == 3 and st["numUsedVgprs"] <= 168, what
+                    elif t["name"] in _WGS_PER_CU:
                         assert st["workgroupsPerCU"] == _WGS_PER_CU[t["name"]], what
                     else:
                         assert t["name"] == "mm_64x64x64_w2x2" and st["workgroupsPerCU"] >= 3, what
@@ -403,3 +405,26 @@ def test_statistics_of_a_planned_gemm_and_tuner_fields(dev):
     mm, best = autotune_matmul(dev, 512, 512, 512, reps=1, use_cache=False, dtype="bf16")
     assert best["vgpr"] and best["vgpr"] <= 512 and best["occupancy"] >= 1 and best["spilling"] == []
     mm.destroy()
+
+
+def test_statistics_are_those_of_the_form_for_three_workgroups(dev):
+    """More than two 128 x 128 tiles a CU run another form of the kernel than fewer do, also where it serves the fused
+    outputs of the tile with K-blocks of 64; what is reported is the one that would be launched."""
+    import ctypes as C
+    from vkgrad_amd import _lib as L
+    from vkgrad_amd.kernels import Matmul
+    cus, buf = dev.compute_units, dev.buffer(1 << 28, "device")
+
+    def reported(tile, rows, **fused):
+        mm, st, ran = Matmul(dev, dtype="bf16", tile=tile, split_k=1), L.KernelStats(), C.c_int()
+        kw = dict(bias=None, accumulate=False, lda=None, ldb=None, ldc=None) | fused
+        ga = mm._args(buf, buf, buf, rows * 128, 1024, 64, 1, (0, 0, 0), **kw)
+        assert dev._lib.mg_kernel_stats_for(dev._ctx, C.byref(ga), C.byref(ran), C.byref(st)) == L.MG_OK
+        return st.wgs_per_cu, ran.value
+
+    full = 2 * cus // 8   # rows of eight tiles, two tiles for a CU
+    assert reported(14, full) == (2, 14) and reported(14, full + 1) == (3, 14)
+    gelu = dict(act="gelu", y16=buf)
+    assert reported(14, full, **gelu) == (2, 14) and reported(14, full + 1, **gelu) == (3, 14)
+    assert reported(3, full, **gelu)[1] == 3 and reported(3, full + 1, **gelu) == (3, 14)
+    buf.destroy()

@@ -415,7 +415,8 @@ def stats_dict(st, tile):
 
 def tile_statistics(dev, tile, layout, dtype="f16", variant=0):
     """statistics() of one instantiation named directly (tile id, layout MG_NN.., dtype,
-    variant 0 aligned / 1 any alignment or bias epilogue / 2 fused activation); None when the
+    variant 0 aligned / 1 any alignment or bias epilogue / 2 fused activation / 3 the same with direct
+    loads, or for three workgroups a CU / 4 aligned, for three workgroups a CU); None when the
     library holds no such instantiation."""
     st = L.KernelStats()
     rc = dev._lib.mg_tile_kernel_stats(dev._ctx, int(tile), int(layout), L.DTYPES[dtype], int(variant), C.byref(st))
