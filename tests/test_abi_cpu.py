@@ -319,6 +319,14 @@ def test_autotuner_times_the_librarys_own_choice(tmp_path, monkeypatch):
     assert K.matmul_from_entry(FakeDev(), e).tile == -1 and K.walk_matters(-1)
 
 
+def test_shipped_plans_do_not_add_slices_with_atomics():
+    """Sums of slices that add into C with atomics have come out short on the device, for a reason not found: K slices of
+    what ships meet in the workspace."""
+    import vkgrad_amd.kernels as K
+    table = K._shipped_table()
+    assert table and not [key for key, e in table.items() if e.get("atomic_split")]
+
+
 def test_plans_tuned_in_context(tmp_path, monkeypatch):
     """kernels.tune_in_context against a deterministic cost: coordinate descent finds plans whose
     merit only shows in the sum (a GEMM that is slower alone but leaves room for its neighbour),
