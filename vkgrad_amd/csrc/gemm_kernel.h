@@ -171,9 +171,8 @@ struct Stage {
 
     u32x4 reg[PER];
     // GENERAL: by how many elements a thread's pieces still have to move (load leaves it to store, one K-block later, so that
-    // nothing waits for a load at its issue), how many of its LDS rows are there, and whether any of this matters
+    // nothing waits for a load at its issue), and how many of its LDS rows are there
     int back, there;
-    bool edge = false;
 
     // Unconditional loads for a K-block that lies entirely inside the matrix in
     // both directions.  `tile` points at the block's first element (uniform over
@@ -181,7 +180,6 @@ struct Stage {
     __device__ __forceinline__ void load_fast(const uint16_t *tile, int64_t ld, int tid) {
         const uint16_t *src = tile + (int64_t)(tid / CPR) * ld + (tid % CPR) * 8;
         const int64_t step = (int64_t)RSTEP * ld;
-        edge = false;
 #pragma unroll
         for (int i = 0; i < PER; i++) {
             if constexpr (GENERAL) reg[i] = *(const u32x4_u *)(src + i * step);
@@ -230,7 +228,6 @@ struct Stage {
     // TAIL: this operand has odd pieces
     template <bool TAIL>
     __device__ __forceinline__ void load_whole(int64_t step_bytes) {
-        edge = false;
         asm("" : "+s"(at));   // a scalar base and lane offsets: the compiler would keep a 64-bit pointer a piece instead
 #pragma unroll
         for (int i = 0; i < PER; i++) reg[i] = *(glb_u32x4_d *)(at + off[i]);
@@ -284,7 +281,6 @@ struct Stage {
     // k0: first k of this block; kend: one past the last valid k for this slice.
     __device__ __forceinline__ void load(const uint16_t *base, int64_t ld, int row0, int nrows,
                                          int k0, int kend, int tid) {
-        edge = GENERAL;
 #pragma unroll
         for (int i = 0; i < PER; i++) {
             const int c = tid + i * NTHREADS;
@@ -327,15 +323,13 @@ struct Stage {
         }
     }
 
-    // FROM 0: whatever load the block came from; 1: load_fast, or load_whole with even pieces; 2: load_whole.
-    template <int FROM = 0, int I = 0>
+    // FROM 1: load_fast, or load_whole with even pieces; 2: load_whole; 3: load.
+    template <int FROM, int I = 0>
     __device__ __forceinline__ void store(uint16_t *lds, int tid) {
         const int c = tid + I * NTHREADS;
         u32x4 *to = (u32x4 *)(lds + c / CPR * PITCH + (c % CPR) * 8);
-        if constexpr (!GENERAL || FROM == 1) *to = reg[I];
-        else if constexpr (FROM == 2) *to = odd_piece<I>(tid);
-        else if (edge) *to = chunk_shift(reg[I], KC || c / CPR < there ? back : 8);
-        else if constexpr (WHOLE) *to = odd_piece<I>(tid);
+        if constexpr (FROM == 2) *to = odd_piece<I>(tid);
+        else if constexpr (FROM == 3 && GENERAL) *to = chunk_shift(reg[I], KC || c / CPR < there ? back : 8);
         else *to = reg[I];
         if constexpr (I + 1 < PER) store<FROM, I + 1>(lds, tid);
     }
@@ -889,6 +883,19 @@ __device__ __forceinline__ void gemm_body(const GemmParams &p, int tile, int sli
             sb.load(B, p.ldb, n0, p.N, kbeg + kb * BK, kend, tid);
         }
     };
+    // What load_block has brought.  One uniform branch for all pieces: a test a piece cost products of few K-blocks 0.1 to 0.5 us each
+    // (backward pass of 315 rows, 192 -> 13 columns 8.5 -> 7.8 us, of 33 rows, 512 -> 10 4.97 -> 4.82; NN 1001 x 1003 x 129 6.9 -> 6.5).  Tiles that lie
+    // inside the matrix, odd pitches and less than two workgroups a CU keep paying for the moves (odd_piece), 60 VALU instructions a K-block:
+    // NN 1152 x 320 x 384 7.3 us, 6.5 with unmoved loads of whole tiles, but 2304 x 640 x 384 8.0, 7.9.
+    auto store_block = [&](uint16_t *to, int kb) {
+        if (kb < nkb_fast) {
+            sa.template store<WHOLE ? 2 : 1>(to, tid);
+            sb.template store<WHOLE ? 2 : 1>(to + SA::ELEMS, tid);
+        } else {
+            sa.template store<3>(to, tid);
+            sb.template store<3>(to + SA::ELEMS, tid);
+        }
+    };
     auto read_frags = [&](const uint16_t *As, int kk, int slot) {
         const uint16_t *Bs = As + SA::ELEMS;
 #pragma unroll
@@ -907,8 +914,7 @@ __device__ __forceinline__ void gemm_body(const GemmParams &p, int tile, int sli
     // (block 0, kk 0) -> af[0], bf[0].
     if (nkb > 0) {
         load_block(0);
-        sa.store(smem, tid);
-        sb.store(smem + SA::ELEMS, tid);
+        store_block(smem, 0);
         if (nkb > 1) load_block(1);
     }
     __syncthreads();
@@ -931,9 +937,11 @@ __device__ __forceinline__ void gemm_body(const GemmParams &p, int tile, int sli
                 read_frags(An, 0, nxt);   // next stage is complete: the barrier below has passed
             }
             if (kk == KK - 2) {
-                if (MODE || kb + 1 < nkb) {
-                    sa.template store<MODE == 0 ? 0 : MODE & 2 ? 2 : 1>(An, tid);
-                    sb.template store<MODE == 0 ? 0 : MODE & 4 ? 2 : 1>(An + SA::ELEMS, tid);
+                if constexpr (MODE) {
+                    sa.template store<MODE & 2 ? 2 : 1>(An, tid);
+                    sb.template store<MODE & 4 ? 2 : 1>(An + SA::ELEMS, tid);
+                } else {
+                    if (kb + 1 < nkb) store_block(An, kb + 1);
                 }
                 if constexpr (MODE) {
                     load_fast(IntC<MODE>{}, kb + 2);
