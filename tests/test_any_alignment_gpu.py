@@ -56,3 +56,24 @@ def test_odd_pieces(dev, layout, tile):
                 assert np.array_equal(bc.download(np.float32, (m, n)), ref), (m, n, k, lda, ldb, shift_a, shift_b, split)
             for x in (ba, bb, bc):
                 x.destroy()
+
+
+@pytest.mark.parametrize("layout,m,n,k,lda,ldb", [
+    ("NN", 5, 70, 130, (1 << 21) + 1, 71), ("NN", 70, 33, 66, 67, 1 << 21), ("NT", 3, 4, 200, (1 << 21) - 1, (1 << 21) + 1),
+    ("TN", 6, 65, 66, (1 << 21) + 3, 65), ("TN", 6, 65, 66, (1 << 21) - 1, 65)])
+def test_pitches_on_both_sides_of_32_bit_offsets(dev, layout, m, n, k, lda, ldb):
+    """Whole K-blocks are loaded at 32-bit offsets from their first dword; pitches of 2^21 elements and more go the careful way."""
+    from vkgrad_amd import _lib as L
+    ta, tb = O.LAYOUTS[layout]
+    a, b = O.make_operands(m, n, k, ta, tb, "bf16", seed=m, integer=True)
+    ref = O.ref_gemm(a, b, ta, tb, "bf16")
+    (ba, at), (bb, bt), bc = _put(dev, a, lda, 1), _put(dev, b, ldb, 1), dev.buffer(m * n * 4, "device")
+    for tile in (3, 4):
+        g = L.GemmArgs()
+        g.struct_size, g.layout, g.dtype, g.tile, g.split_k = C.sizeof(L.GemmArgs), LAYOUT_ID[layout], 1, tile, 1
+        g.m, g.n, g.k, g.a, g.b, g.c, g.lda, g.ldb, g.ldc, g.nbatch = m, n, k, at, bt, bc.ptr, lda, ldb, n, 1
+        bc.upload(np.full((m, n), np.nan, np.float32))
+        assert dev._lib.mg_gemm(dev._ctx, C.byref(g)) == 0
+        assert np.array_equal(bc.download(np.float32, (m, n)), ref), tile
+    for x in (ba, bb, bc):
+        x.destroy()
