@@ -228,10 +228,16 @@ struct Stage {
     // TAIL: this operand has odd pieces
     template <bool TAIL>
     __device__ __forceinline__ void load_whole(int64_t step_bytes) {
-        asm("" : "+s"(at));   // a scalar base and lane offsets: the compiler would keep a 64-bit pointer a piece instead
+        asm("" : "+s"(at));   // a scalar base and 32-bit lane offsets: the compiler would keep a 64-bit pointer or offset a piece instead
 #pragma unroll
-        for (int i = 0; i < PER; i++) reg[i] = *(glb_u32x4_d *)(at + off[i]);
-        if constexpr (TAIL && !KC) tail = *(glb_u32_t *)(at + toff);
+        for (int i = 0; i < PER; i++) {
+            asm("" : "+v"(off[i]));
+            reg[i] = *(glb_u32x4_d *)(at + off[i]);
+        }
+        if constexpr (TAIL && !KC) {
+            asm("" : "+v"(toff));
+            tail = *(glb_u32_t *)(at + toff);
+        }
         at += step_bytes;
     }
     template <int I>
@@ -884,9 +890,9 @@ __device__ __forceinline__ void gemm_body(const GemmParams &p, int tile, int sli
         }
     };
     // What load_block has brought.  One uniform branch for all pieces: a test a piece cost products of few K-blocks 0.1 to 0.5 us each
-    // (backward pass of 315 rows, 192 -> 13 columns 8.5 -> 7.8 us, of 33 rows, 512 -> 10 4.97 -> 4.82; NN 1001 x 1003 x 129 6.9 -> 6.5).  Tiles that lie
+    // (backward pass of 315 rows, 192 -> 13 columns 8.5 -> 7.9 us, of 33 rows, 512 -> 10 4.97 -> 4.81; NN 1001 x 1003 x 129 6.9 -> 6.5).  Tiles that lie
     // inside the matrix, odd pitches and less than two workgroups a CU keep paying for the moves (odd_piece), 60 VALU instructions a K-block:
-    // NN 1152 x 320 x 384 7.3 us, 6.5 with unmoved loads of whole tiles, but 2304 x 640 x 384 8.0, 7.9.
+    // NN 1152 x 320 x 384 7.1 us, 6.5 with unmoved loads of whole tiles, but 2304 x 640 x 384 7.8, 7.9.
     auto store_block = [&](uint16_t *to, int kb) {
         if (kb < nkb_fast) {
             sa.template store<WHOLE ? 2 : 1>(to, tid);
